@@ -399,6 +399,80 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
   return gemm_lds_bytes(fmt, q, static_cast<int>(k)) <= kLdsMax;
 }
 
+// The tiled GEMM (gemm_tile.h) takes the larger batches, where its staged activations pay.  Measured on MI355X against
+// gemm.hip's kernel (graph replays) over 9 shapes (127 x 4096 to 28672 x 4096) and 12 column counts: from 25 columns on
+// it is 1.9 times as fast in the geometric mean, at best 5.3 times (Q4_0 14336 x 4096 at 512 columns 385 -> 119 us, TQ2_0
+// 6912 x 2560 at 2048 columns 326 -> 67, Q4_K 4096 x 14336 at 1001 columns 561 -> 215); up to 24 (Q4_K: 48) columns
+// gemm.hip's kernel, which unpacks fewer activations and splits K 8 ways, is as fast or faster (Q4_K 4096 x 14336 at 32
+// columns 23.6 against 27.9 us), and so it is on rows of at most 4 K steps, which are over before the tile's staging
+// pays.
+//
+// The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
+// round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
+// launch has 3 us besides.  The constants are a least-squares fit over those shapes (estimates within 2-6% in the
+// median), and the plan they pick is within 1.2% of the fastest one in the geometric mean (at worst 16%).
+struct TileCost {
+  TilePlan p;
+  int slots;
+  float ab[3][2];  // (a, b): Q4_0 and IQ4_NL, TQ2_0, Q8_0
+};
+constexpr TileCost kTileCosts[] = {
+    {{1, 1, 1, 8}, 2, {{0.f, 0.80f}, {0.f, 0.82f}, {0.f, 0.99f}}},
+    {{1, 2, 1, 4}, 4, {{0.12f, 0.57f}, {0.01f, 0.59f}, {0.05f, 0.81f}}},
+    {{2, 1, 2, 4}, 2, {{0.23f, 0.75f}, {0.f, 0.82f}, {0.03f, 1.02f}}},
+    {{2, 1, 4, 4}, 1, {{0.f, 1.71f}, {0.f, 1.59f}, {0.f, 2.01f}}},
+    {{4, 1, 4, 2}, 2, {{0.28f, 0.96f}, {0.10f, 0.90f}, {0.28f, 1.10f}}},
+    {{4, 2, 4, 1}, 3, {{0.61f, 0.71f}, {0.26f, 0.70f}, {0.69f, 0.83f}}},
+    {{4, 2, 8, 1}, 2, {{1.15f, 1.14f}, {0.31f, 1.33f}, {1.31f, 1.30f}}},
+    {{4, 2, 8, 2}, 1, {{0.f, 3.91f}, {0.f, 2.95f}, {0.f, 4.38f}}},
+};
+// Q4_K's waves also hold a block's first half of every output, so its large tiles are half as tall.
+constexpr TileCost kTileCostsQ4K[] = {
+    {{1, 1, 1, 8}, 2, {{0.24f, 0.73f}}}, {{1, 2, 1, 4}, 4, {{0.41f, 0.55f}}}, {{2, 1, 2, 4}, 2, {{0.44f, 0.69f}}},
+    {{2, 1, 4, 4}, 1, {{0.f, 1.77f}}},   {{4, 1, 4, 2}, 1, {{0.f, 1.36f}}},   {{4, 1, 8, 2}, 1, {{0.f, 2.09f}}},
+    {{4, 2, 4, 1}, 2, {{0.41f, 0.73f}}}, {{8, 1, 8, 1}, 1, {{0.f, 1.75f}}},
+};
+
+// False when the call stays on gemm.hip's kernel: few columns, short rows, or past the tile's 32-bit buffer offsets
+// (128 rows of SW bytes, 128 columns of K) or the grid's column groups.
+bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePlan* p) {
+  const int64_t nblk = k / fmt_info(fmt).block;
+  const int64_t steps = fmt == FMT_Q4_K ? 2 * nblk : fmt == FMT_TQ2_0 ? nblk : (nblk + 3) / 4;
+  if (m <= (fmt == FMT_Q4_K ? 48 : 24) || steps <= 4 || n < 1) return false;
+  // Q4_K's 49-64 columns over at most 3 row tiles a CU: 4096 x 14336 40 us here and there, 6912 x 2560 17.5 -> 14.1 but
+  // 4096 x 4096 15.1 either way; over more, 14336 x 4096 45.1 -> 28.5 us, 28672 x 4096 89 -> 42
+  if (fmt == FMT_Q4_K && m <= 64 && n <= 48 * static_cast<int64_t>(device_cus())) return false;
+  if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
+  const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : 0;
+  const int64_t cus = device_cus();
+  double best = -1;
+  for (const TileCost& t : fmt == FMT_Q4_K ? kTileCostsQ4K : kTileCosts) {
+    const int64_t groups = (m + 16 * t.p.cn - 1) / (16 * t.p.cn);
+    if (groups > 65535) continue;
+    const int64_t wgs = (n + 16 * t.p.wn * t.p.rw - 1) / (16 * t.p.wn * t.p.rw) * groups;
+    const int64_t load = (wgs + cus - 1) / cus;  // workgroups on the fullest CU
+    const int64_t per = fmt == FMT_Q4_K ? 2 * ((nblk + t.p.wk - 1) / t.p.wk) : (steps + t.p.wk - 1) / t.p.wk;
+    const double rounds = load > t.slots ? static_cast<double>(load) / t.slots : 1.0;
+    const double us = per * (t.ab[row][0] * rounds + t.ab[row][1] * static_cast<double>(load));
+    if (best < 0 || us < best) {
+      best = us;
+      *p = t.p;
+    }
+  }
+  return best >= 0;
+}
+
+hipError_t launch_gemm_tile(const GemmCall& c, const TilePlan& p, hipStream_t stream) {
+  switch (c.fmt) {
+    case FMT_Q4_0: return launch_gemm_tile_q4(c, p, stream);
+    case FMT_IQ4_NL: return launch_gemm_tile_iq4(c, p, stream);
+    case FMT_Q8_0: return launch_gemm_tile_q8(c, p, stream);
+    case FMT_TQ2_0: return launch_gemm_tile_tq2(c, p, stream);
+    case FMT_Q4_K: return launch_gemm_tile_q4k(c, p, stream);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 // The matrix-core GEMV (gemv_tq2_mfma.hip) for kMfmaM TQ2_0 columns, block_n == 0 in dp4a mode.  Measured on MI355X
 // against the lean kernel's plans (graph replays, cold weights), three columns with q8_K in: BitNet-2B 6912 x 2560
 // 3.95 -> 3.84 us, 2560 x 6912 4.44 -> 4.22, 6913 x 2816 4.5 -> 3.9, 4097 x 2816 4.2 -> 3.3, 32768 x 8192 23.3 ->
@@ -530,7 +604,11 @@ int gemv_entry(int fmt, bool fused, const char* name, const GemvArgs& a, int64_t
           c.n = static_cast<int>(mats[i].n);
           c.k = static_cast<int>(K);
           c.sw = mats[i].sw;
-          const int st = hip_status(launch_gemm(c, gp, static_cast<hipStream_t>(stream)), name);
+          TilePlan tp;
+          const int st = hip_status(gemm_tile_plan(fmt, mc, c.n, K, c.sw, &tp)
+                                        ? launch_gemm_tile(c, tp, static_cast<hipStream_t>(stream))
+                                        : launch_gemm(c, gp, static_cast<hipStream_t>(stream)),
+                                    name);
           if (st != KOMP_OK) return st;
         }
       }
@@ -784,6 +862,8 @@ int komp_gemm_plan(int fmt, int64_t M, int64_t N, int64_t K, int64_t SW, int* ro
   GemmPlan p;
   if (!gemm_plan(fmt, M < kGemmMaxCols ? M : kGemmMaxCols, N, K, SW, &p))
     return fail(KOMP_EINVAL, "komp_gemm_plan: K=%lld / SW=%lld past the GEMM's limits", (long long)K, (long long)SW);
+  TilePlan t;
+  if (gemm_tile_plan(fmt, M < kGemmMaxCols ? M : kGemmMaxCols, N, K, SW, &t)) p = GemmPlan{t.wk, t.rw, t.wn, t.cn, 1};
   if (rows_per_wg != nullptr) *rows_per_wg = 16 * p.wn * p.wr;
   if (cols_per_wg != nullptr) *cols_per_wg = 16 * p.cn;
   if (waves != nullptr) *waves = p.wk * p.wr;

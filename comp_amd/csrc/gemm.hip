@@ -3,7 +3,8 @@
 //   Y[m][n] = sum_b d_w(n, b) * d_x(m, b) * s(m, n, b),  s = the exact int32 dot of weight block b of row n with
 //   activation block b of column m,
 // and the same optional S [M][N][K/block] of exact block dots.  The GEMVs stream the weights once per 1..3 columns;
-// this kernel streams them once per 64 columns, so a batch of decode tokens reads each weight byte once.
+// this kernel streams them once per 64 columns, so a batch of decode tokens reads each weight byte once.  Larger batches
+// and prompts run the tiled kernel of gemm_tile.h (gemm_tile_plan in abi.hip says from where).
 //
 // Tiles.  A workgroup (W waves) owns 16*WN weight rows x 16*CN activation columns and all of K.  Its waves split K:
 // a K step is 64 contiguous bytes of each weight row (4 Q4_0 blocks or 1 TQ2_0 block) and wave w takes steps

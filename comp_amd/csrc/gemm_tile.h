@@ -1,0 +1,641 @@
+// Tiled matrix-core GEMM for many activation columns (prompts, large batches): the result definition, arguments and
+// optional S of gemm.hip's kernel, with the activations staged once per workgroup in LDS, in the form the matrix
+// instruction takes, instead of read and rearranged by every wave.
+//
+// Bound.  Each block's exact integer dot is scaled in f32 by its own d_w * d_x, so the VALU runs a fixed number of
+// instructions per output and block beside the matrix cores.  The batched kernel in gemm.hip spends per 16x16 tile and
+// 32-value block 12 of them on the scaling (convert, multiply, fused multiply-add of 4 outputs a lane) and about as
+// many on rearranging operands, re-read per 64 columns.  Here:
+//   32-value blocks (Q4_0, IQ4_NL, Q8_0) and Q4_K go through v_mfma_f32_16x16x32_f16 with both operands as integers in
+//     f16.  Every product and partial sum is an integer below 2^24 (Q8_0: 32 * 128 * 128 = 2^19; Q4_K: the 6-bit
+//     sub-block scale times the nibble, at most 945, over half a block: 945 * 128 * 128 = 15.5 M; the two halves are
+//     added in f32, which rounds where the integer sum's conversion would), so the f32 result is the exact block dot,
+//     whatever order the matrix core adds in, and needs no conversion: 8 instructions instead of
+//     12.  One f16 instruction covers a 32-value block in the time the int8 one does (its int8 form of K 32 has no
+//     higher rate).
+//   TQ2_0's 256-value blocks stay on v_mfma_i32_16x16x64_i8 (twice the f16 rate; the scaling is 1/8 as often).
+//
+// Tile.  A workgroup of WK x RW waves owns 16*WN*RW weight rows x 16*CN columns.  The waves of a K group split its rows
+// (each unpacks its own weights from registers, no wave twice) and share its staged activations; the WK groups take
+// contiguous K ranges and add their partial sums at the end in group order.  A K step is 64 bytes of each weight row
+// (Q8_0: 128): 128 values (TQ2_0: 256).  Two LDS buffers: during step i every thread unpacks its share of step i+1's
+// activations (loaded a step earlier) into the other buffer, so one barrier a step suffices and every global load has a
+// whole step to arrive.
+//
+// LDS.  Operand unit (piece, group g) of a column is 16 bytes; units lie [piece][g][column ^ g], so a fragment read
+// covers 256 contiguous, aligned bytes per 16 lanes (a permutation of 4 columns within it).  The staging writes several
+// pieces (TQ2_0: and groups) of one column at a time: a pad of 64 bytes after each piece and the column's low bits
+// crossed with g put those on different banks.  (Padding every unit row by 16 bytes instead left the reads with 42% of
+// their LDS cycles in conflicts.)
+#pragma once
+
+#include <hip/hip_ext.h>
+
+#include <type_traits>
+
+#include "komp_device.h"
+#include "komp_internal.h"
+
+namespace komp {
+namespace gemm_tile {
+
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kRsrcWord3 = 0x00020000;  // buffer descriptor word 3 on gfx9: 32-bit data, no swizzle
+constexpr unsigned kOob = 0x7FFFFFF0u;  // an offset past every descriptor's range: the load returns zeros
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
+  const int n = static_cast<int>(bytes <= 0 ? 0 : (bytes < 0x7FFFFFF0 ? bytes : 0x7FFFFFF0));
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, kRsrcWord3);
+}
+
+// 4x4 dword transpose across the four 16-lane rows of a wave: on entry row g of v[q] holds element (q, g), on exit row
+// g of t[j] holds element (g, j).
+__device__ __forceinline__ void transpose4(const u32x4& v, unsigned (&t)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  t[0] = c[0];
+  t[1] = c[1];
+  t[2] = d[0];
+  t[3] = d[1];
+}
+
+__device__ __forceinline__ f16x2 as_h2(unsigned v) { return __builtin_bit_cast(f16x2, v); }
+__device__ __forceinline__ unsigned as_u(f16x2 v) { return __builtin_bit_cast(unsigned, v); }
+__device__ __forceinline__ f16x2 h2(float a) { return f16x2{static_cast<_Float16>(a), static_cast<_Float16>(a)}; }
+
+// The four signed bytes of q as f16 integers: bytes 0 and 2 in e, bytes 1 and 3 in o (the order the nibble forms give).
+__device__ __forceinline__ void bytes_to_f16(unsigned q, unsigned& e, unsigned& o) {
+  const unsigned u = q ^ 0x80808080u;  // byte + 128
+  e = as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04020400u)) - h2(1152.f));
+  o = as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030401u)) - h2(1152.f));
+}
+
+__device__ __forceinline__ f16x8 frag(unsigned a, unsigned b, unsigned c, unsigned d) {
+  return __builtin_bit_cast(f16x8, u32x4{a, b, c, d});
+}
+
+// LDS bytes of one K group's part: two activation buffers, two d_x buffers and (Q4_K) two buffers of 16-value sums; and
+// of one wave's scales.
+template <int FMT, int CN>
+struct Lds {
+  static constexpr int kRow = 16 * CN * 16;                // a unit row: 16 bytes a column
+  static constexpr int kPiece = 4 * kRow + 64;             // the four groups' rows of a piece, and the pad
+  static constexpr int kBuf = 4 * kPiece;
+  static constexpr int kDx = 16 * CN * (FMT == FMT_TQ2_0 || FMT == FMT_Q4_K ? 1 : 4) * 4;
+  static constexpr int kSums = FMT == FMT_Q4_K ? 2 * kRow : 0;
+  static constexpr int kGroup = 2 * (kBuf + kDx + kSums);
+  static constexpr int scales(int wn) {  // f32 per wave: 4 blocks of 16 rows a tile; TQ2_0 one; Q4_K d and dmin
+    return wn * 16 * (FMT == FMT_TQ2_0 ? 1 : FMT == FMT_Q4_K ? 2 : 4) * 4;
+  }
+};
+
+template <int FMT, int RW, int WN, int CN, int WK>
+constexpr size_t lds_bytes() {
+  const size_t stage = static_cast<size_t>(WK) * Lds<FMT, CN>::kGroup + WK * RW * Lds<FMT, CN>::scales(WN);
+  const size_t red = static_cast<size_t>(WK - 1) * RW * WN * CN * 4 * 64 * 4;
+  return stage > red ? stage : red;
+}
+
+template <int FMT, int RW, int WN, int CN, int WK, int DW, bool STORE_S>
+__global__ void __launch_bounds__(64 * RW * WK, RW * WK == 4 ? 2 : 1)
+tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __restrict__ WQ,
+                 const int16_t* __restrict__ WS, const int8_t* __restrict__ XQ, const float* __restrict__ XD,
+                 float* __restrict__ Y, int32_t* __restrict__ S) {
+  constexpr bool NIB4 = FMT == FMT_Q4_0 || FMT == FMT_IQ4_NL;
+  constexpr bool Q8 = FMT == FMT_Q8_0;
+  constexpr bool BLK32 = NIB4 || Q8;
+  constexpr bool TQ2 = FMT == FMT_TQ2_0;
+  constexpr bool QK = FMT == FMT_Q4_K;
+  using L = Lds<FMT, CN>;
+  constexpr int T = 64 * RW;          // threads of a K group
+  constexpr int COLS = 16 * CN;
+  constexpr int WGR = 16 * WN * RW;   // rows of the workgroup
+  constexpr int WV = Q8 ? 2 : 1;      // 16-byte weight loads per row tile and step
+  constexpr int XB = TQ2 ? 256 : 128;  // activation bytes per column and step
+  constexpr int BI = TQ2 ? COLS * 16 / T : COLS * 4 / T;  // staging items a thread: 16 bytes (TQ2_0) or 32
+  static_assert(BI * T == (TQ2 ? COLS * 16 : COLS * 4), "the threads split the staged columns evenly");
+  extern __shared__ __align__(16) unsigned char lds[];
+  // kBias in a VGPR, so that masking a nibble pair and putting the bias on is one v_and_or_b32 (which takes one literal)
+  unsigned bias;
+  asm("v_mov_b32 %0, 0x64006400" : "=v"(bias));
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave / RW;   // K group
+  const int wr = wave % RW;   // row group
+  const int tid = threadIdx.x - wk * T;
+  const int r16 = lane & 15;
+  const int g = lane >> 4;
+  const int n0 = blockIdx.x * WGR;
+  if (n0 >= N) return;  // a padding workgroup: the whole workgroup leaves before any barrier
+  const int nw = n0 + 16 * WN * wr;
+  const int m0 = blockIdx.y * COLS;
+  const int rows = max(0, min(16 * WN, N - nw));
+  const int cols = min(COLS, M - m0);
+  const int nsteps = QK ? 2 * nblk : (TQ2 ? nblk : (nblk + 3) / 4);
+  const int per = QK ? 2 * ((nblk + WK - 1) / WK) : (nsteps + WK - 1) / WK;  // steps a K group (the same for all)
+  const int s0 = wk * per;
+  const int s1 = min(nsteps, s0 + per);
+
+  unsigned char* const gl = lds + wk * L::kGroup;
+  unsigned char* const dxl = gl + 2 * L::kBuf;
+  unsigned char* const suml = dxl + 2 * L::kDx;
+  float* const scl = reinterpret_cast<float*>(lds + WK * L::kGroup + wave * L::scales(WN));
+
+  const auto wq = rsrc(WQ + nw * SW, rows * SW);
+  const auto ws = rsrc(WS + static_cast<int64_t>(nw) * nblk * (QK ? 8 : 1),
+                       static_cast<int64_t>(rows) * nblk * (QK ? 16 : 2));
+  const auto xq = rsrc(XQ + static_cast<int64_t>(m0) * K, static_cast<int64_t>(cols) * K);
+  const auto xd = rsrc(XD + static_cast<int64_t>(m0) * nblk, static_cast<int64_t>(cols) * nblk * 4);
+
+  // ---- global loads, a step's worth each ----
+  unsigned va[WN], vs[WN];
+#pragma unroll
+  for (int t = 0; t < WN; ++t) {
+    va[t] = static_cast<unsigned>((16 * t + r16) * SW + 16 * g);
+    vs[t] = static_cast<unsigned>((16 * t + r16) * nblk * (QK ? 16 : 2));
+  }
+  unsigned vx[BI], lx[BI];  // an item's source offset and its LDS offset
+#pragma unroll
+  for (int i = 0; i < BI; ++i) {
+    const int idx = i * T + tid;
+    if constexpr (TQ2) {  // 16 bytes q of a column: half q/8, crumb (q%8)/2, 16-byte half q%2 of the 32
+      const int q = idx & 15, c = idx >> 4;
+      vx[i] = static_cast<unsigned>(c * K + 16 * q);
+      const int j = (q & 7) >> 1, gq = (q >> 3) * 2 + (q & 1);
+      lx[i] = static_cast<unsigned>(j * L::kPiece + gq * L::kRow + 16 * (c ^ gq));
+    } else {  // block j of a column
+      const int j = idx & 3, c = idx >> 2;
+      vx[i] = static_cast<unsigned>(c * K + 32 * j);
+      lx[i] = static_cast<unsigned>(j * L::kPiece + 16 * c);
+    }
+  }
+  struct Weights {  // one step's weights and scales of the wave's rows
+    u32x4 a[WN][WV];
+    u32x4 e[QK ? WN : 1];        // Q4_K: the block's 16 scale-plane bytes
+    unsigned short h[QK ? 1 : WN];
+  };
+  Weights wring[DW];
+  auto load_w = [&](Weights& w, int s) {
+    const unsigned off = s < s1 ? 64u * WV * s : kOob;
+#pragma unroll
+    for (int t = 0; t < WN; ++t) {
+#pragma unroll
+      for (int v = 0; v < WV; ++v)
+        w.a[t][v] = __builtin_amdgcn_raw_buffer_load_b128(wq, va[t] + off + 64 * v, 0, 0);
+      if constexpr (QK)
+        w.e[t] = __builtin_amdgcn_raw_buffer_load_b128(ws, vs[t] + (s < s1 ? 16u * (s >> 1) : kOob), 0, 0);
+      else if constexpr (TQ2)
+        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 ? 2u * s : kOob), 0, 0);
+      else  // a block past K has scale zero
+        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 && 4 * s + g < nblk ? 8u * s + 2u * g : kOob),
+                                                       0, 0);
+    }
+  };
+  constexpr int XV = TQ2 ? 1 : 2;
+  constexpr int DI = BLK32 ? BI : (COLS + T - 1) / T;
+  struct Acts {  // one step's activations, this thread's share
+    u32x4 x[BI][XV];
+    float d[DI];
+  };
+  Acts xraw;
+  auto load_x = [&](Acts& a, int s) {
+    const unsigned off = s < s1 ? static_cast<unsigned>(XB) * s : kOob;
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int v = 0; v < XV; ++v)
+        a.x[i][v] = __builtin_amdgcn_raw_buffer_load_b128(xq, vx[i] + off + 16 * v, 0, 0);
+#pragma unroll
+    for (int i = 0; i < DI; ++i) {
+      const int idx = i * T + tid;
+      unsigned o;
+      if constexpr (BLK32)
+        o = s < s1 && 4 * s + (idx & 3) < nblk ? static_cast<unsigned>((idx >> 2) * nblk + 4 * s + (idx & 3)) * 4u : kOob;
+      else
+        o = s < s1 && idx < COLS ? static_cast<unsigned>(idx * nblk + (QK ? s >> 1 : s)) * 4u : kOob;
+      a.d[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xd, o, 0, 0));
+    }
+  };
+  // step s's activations from the registers into LDS buffer s & 1
+  auto stage = [&](const Acts& a, int s) {
+    unsigned char* const b = gl + ((s - s0) & 1) * L::kBuf;
+    float* const dxb = reinterpret_cast<float*>(dxl + ((s - s0) & 1) * L::kDx);
+#pragma unroll
+    for (int i = 0; i < BI; ++i) {
+      if constexpr (TQ2) {
+        *reinterpret_cast<u32x4*>(b + lx[i]) = a.x[i][0];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // group q: values 4q..4q+3 and 16+4q..16+4q+3
+          u32x4 u;
+          unsigned e, o;
+          bytes_to_f16(a.x[i][0][q], e, o);
+          u[0] = e;
+          u[1] = o;
+          bytes_to_f16(a.x[i][1][q], e, o);
+          u[2] = e;
+          u[3] = o;
+          *reinterpret_cast<u32x4*>(b + (lx[i] ^ (16 * q)) + q * L::kRow) = u;
+        }
+        if constexpr (QK) {  // the item's two 16-value sums (at most 16 * 128: exact in f16)
+          const int idx = i * T + tid;
+          int lo = 0, hi = 0;
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            lo = __builtin_amdgcn_sdot4(static_cast<int>(a.x[i][0][q]), 0x01010101, lo, false);
+            hi = __builtin_amdgcn_sdot4(static_cast<int>(a.x[i][1][q]), 0x01010101, hi, false);
+          }
+          const f16x2 p = {static_cast<_Float16>(static_cast<float>(lo)), static_cast<_Float16>(static_cast<float>(hi))};
+          *reinterpret_cast<unsigned*>(suml + (((s - s0) >> 1) & 1) * L::kSums + (s & 1) * L::kRow + 16 * (idx >> 2) +
+                                       4 * (idx & 3)) = as_u(p);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DI; ++i) {
+      const int idx = i * T + tid;
+      if (BLK32 || DI * T == COLS || idx < COLS) dxb[idx] = a.d[i];  // BLK32: [column][block of the step]
+    }
+  };
+
+  f32x4 acc[WN][CN];
+#pragma unroll
+  for (int t = 0; t < WN; ++t)
+#pragma unroll
+    for (int u = 0; u < CN; ++u) acc[t][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  f32x4 half[QK ? WN : 1][QK ? CN : 1];  // Q4_K: the dots of a block's first half
+
+  auto store_s = [&](const f32x4& v, int t, int u, int b, int stride, int at, bool add) {
+    const int col = m0 + 16 * u + r16;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int row = nw + 16 * t + 4 * g + r;
+      if (col < M && row < N) {
+        int32_t* p = S + ((static_cast<int64_t>(col) * N + row) * nblk + b) * stride + at;
+        const int x = static_cast<int>(v[r]);
+        *p = add ? *p + x : x;
+      }
+    }
+  };
+
+  // The step's products run as a pipeline over (piece, column tile): the operand fragments are read from LDS two tiles
+  // ahead, and a tile's result is scaled while the next tile's matrix instruction runs.  The scheduling barriers keep
+  // that order (left alone, the compiler scales each result right behind its matrix instruction and waits for it), and
+  // the empty asm statements pin each sum's update to its place (otherwise it may be moved down to the sum's next use, a
+  // step later, with every result of the step kept live: 1000 bytes a lane of spills).
+  auto compute = [&](const Weights& w, int s, auto odd) {
+    const unsigned char* const b = gl + ((s - s0) & 1) * L::kBuf + (r16 ^ g) * 16 + g * L::kRow;
+    const unsigned char* const dxp = dxl + ((s - s0) & 1) * L::kDx;
+    if constexpr (BLK32) {
+      constexpr int NI = 4 * CN;  // i = j * CN + u: block j of the step, column tile u
+      unsigned ta[WN][WV][4];
+#pragma unroll
+      for (int t = 0; t < WN; ++t)
+#pragma unroll
+        for (int v = 0; v < WV; ++v) transpose4(w.a[t][v], ta[t][v]);
+      f16x8 a[2][WN], x[4];
+      f32x4 dw[2][WN], cc[2][WN], dx[CN];
+      auto fetch = [&](int i) {
+        x[i & 3] = *reinterpret_cast<const f16x8*>(b + (i / CN) * L::kPiece + 256 * (i % CN));
+      };
+      auto unpack = [&](int j) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          if constexpr (FMT == FMT_Q4_0) {
+            const unsigned p = ta[t][0][j], q = p >> 8;
+            a[j & 1][t] =
+                frag(as_u(as_h2((p & 0x000F000Fu) | bias) - h2(1032.f)), as_u(as_h2((q & 0x000F000Fu) | bias) - h2(1032.f)),
+                     as_u(__builtin_elementwise_fma(as_h2((p & 0x00F000F0u) | bias), h2(0.0625f), h2(-72.f))),
+                     as_u(__builtin_elementwise_fma(as_h2((q & 0x00F000F0u) | bias), h2(0.0625f), h2(-72.f))));
+          } else {
+            unsigned lo, hi, e0, o0, e1, o1;
+            if constexpr (FMT == FMT_IQ4_NL) {
+              iq4_nl_lut(ta[t][0][j], lo, hi);
+            } else {
+              lo = ta[t][j >> 1][2 * (j & 1)];
+              hi = ta[t][j >> 1][2 * (j & 1) + 1];
+            }
+            bytes_to_f16(lo, e0, o0);
+            bytes_to_f16(hi, e1, o1);
+            a[j & 1][t] = frag(e0, o0, e1, o1);
+          }
+          dw[j & 1][t] = *reinterpret_cast<const f32x4*>(scl + (t * 4 + j) * 16 + 4 * g);
+        }
+      };
+      auto scale = [&](int i) {
+        const int j = i / CN, u = i % CN;
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          if (STORE_S && 4 * s + j < nblk && s < s1) store_s(cc[i & 1][t], t, u, 4 * s + j, 1, 0, false);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            acc[t][u][r] = __builtin_fmaf(cc[i & 1][t][r] * dw[j & 1][t][r], dx[u][j], acc[t][u][r]);
+          asm volatile("" : "+v"(acc[t][u]));
+        }
+      };
+      fetch(0);
+      fetch(1);
+#pragma unroll
+      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const f32x4*>(dxp + (16 * u + r16) * 16);
+      unpack(0);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int j = i / CN;
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < NI) fetch(i + 2);
+#pragma unroll
+        for (int t = 0; t < WN; ++t)
+          cc[i & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j & 1][t], x[i & 3], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (i > 0) scale(i - 1);
+        if (i % CN == CN - 1 && j < 3) unpack(j + 1);
+      }
+      scale(NI - 1);
+    } else if constexpr (TQ2) {
+      i32x4 a[WN][4], x[2][4], cc[2][WN];
+      f32x4 dw[WN];
+      float dx[CN];
+      auto fetch = [&](int u) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) x[u & 1][v] = *reinterpret_cast<const i32x4*>(b + v * L::kPiece + 256 * u);
+      };
+      auto scale = [&](int u) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          f32x4 cf;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) cf[r] = static_cast<float>(cc[u & 1][t][r]);
+          if (STORE_S && s < s1) store_s(cf, t, u, s, 1, 0, false);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][u][r] = __builtin_fmaf(dx[u] * dw[t][r], cf[r], acc[t][u][r]);
+          asm volatile("" : "+v"(acc[t][u]));
+        }
+      };
+      fetch(0);
+#pragma unroll
+      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+#pragma unroll
+      for (int t = 0; t < WN; ++t) {
+        dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 16 + 4 * g);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int d = 0; d < 4; ++d)  // crumbs 0..3 -> -1, 0, 1, 2 (a byte table lookup)
+            a[t][v][d] = static_cast<int>(
+                __builtin_amdgcn_perm(0, 0x020100FFu, (w.a[t][0][d] >> (2 * v)) & 0x03030303u));
+      }
+#pragma unroll
+      for (int u = 0; u < CN; ++u) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (u + 1 < CN) fetch(u + 1);
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int t = 0; t < WN; ++t)
+            cc[u & 1][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[t][v], x[u & 1][v],
+                                                                 v == 0 ? i32x4{0, 0, 0, 0} : cc[u & 1][t], 0, 0, 0);
+        if (u > 0) scale(u - 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      scale(CN - 1);
+    } else {
+      // Q4_K: half s % 2 of block s / 2, sub-blocks i = 0..3 of the half: the low (even i) or high nibbles of pieces
+      // 2(i/2), 2(i/2) + 1.  The operand is scale * nibble (at most 945), so the half's four sub-blocks run one chain;
+      // the block's mins term takes one more instruction over its 16 sums of 16 activations, at the odd half.
+      constexpr bool hb = decltype(odd)::value;
+      constexpr int NF = hb ? 5 : 4;  // operand fragments a column tile: four sub-blocks and (odd half) the sums
+      constexpr int NI = NF * CN;
+      f16x8 a[WN][4], x[4];
+      f32x4 dw[WN], dm[WN], cc[2][WN], cm[hb ? 2 : 1][WN];
+      f16x8 am[WN];
+      float dx[CN];
+      const unsigned char* const sp = suml + (((s - s0) >> 1) & 1) * L::kSums + (g & 1) * L::kRow + r16 * 16;
+      auto fetch = [&](int i) {
+        const int u = i / NF, f = i % NF;
+        x[i & 3] = *reinterpret_cast<const f16x8*>(f < 4 ? b + f * L::kPiece + 256 * u : sp + 256 * u);
+      };
+      auto scale = [&](int u) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          if constexpr (!hb) {
+            half[t][u] = cc[u & 1][t];
+            asm volatile("" : "+v"(half[t][u]));
+          } else {
+            // the block's sd: a sum of two exact integers, rounded once as the integer's conversion would be
+            if constexpr (STORE_S) {
+              if (s < s1) {
+                store_s(half[t][u], t, u, s >> 1, 2, 0, false);
+                store_s(cc[u & 1][t], t, u, s >> 1, 2, 0, true);
+                store_s(cm[u & 1][t], t, u, s >> 1, 2, 1, false);
+              }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float sd = half[t][u][r] + cc[u & 1][t][r];
+              acc[t][u][r] += __builtin_fmaf(sd, dw[t][r] * dx[u], -cm[u & 1][t][r] * (dm[t][r] * dx[u]));
+            }
+            asm volatile("" : "+v"(acc[t][u]));  // as above
+          }
+        }
+      };
+      fetch(0);
+      fetch(1);
+#pragma unroll
+      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+#pragma unroll
+      for (int t = 0; t < WN; ++t) {
+        unsigned ta[4];
+        transpose4(w.a[t][0], ta);
+        if constexpr (hb) dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 4 * g);
+        if constexpr (hb) dm[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 16 + 4 * g);
+        const u32x4 e = w.e[t];
+        const unsigned sc = hb ? (e[3] & 0x0F0F0F0Fu) | ((e[1] >> 2) & 0x30303030u) : e[1] & 0x3F3F3F3Fu;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          constexpr unsigned kSel[4] = {0x04000400u, 0x04010401u, 0x04020402u, 0x04030403u};
+          // (1024 + s) - 1024: the scale in both halves; then 1024 + q times it, less 1024 times it (odd i: 16 q)
+          const f16x2 f = as_h2(__builtin_amdgcn_perm(0x64646464u, sc, kSel[i])) - h2(1024.f);
+          const f16x2 m = (i & 1) ? f * h2(0.0625f) : f;
+          const f16x2 k = f * h2((i & 1) ? -64.f : -1024.f);
+          const unsigned mask = (i & 1) ? 0x00F000F0u : 0x000F000Fu;
+          const unsigned p0 = ta[2 * (i >> 1)], p1 = ta[2 * (i >> 1) + 1];
+          a[t][i] = frag(as_u(__builtin_elementwise_fma(as_h2((p0 & mask) | bias), m, k)),
+                         as_u(__builtin_elementwise_fma(as_h2(((p0 >> 8) & mask) | bias), m, k)),
+                         as_u(__builtin_elementwise_fma(as_h2((p1 & mask) | bias), m, k)),
+                         as_u(__builtin_elementwise_fma(as_h2(((p1 >> 8) & mask) | bias), m, k)));
+        }
+        // slot e of groups 0 and 1: the min of sub-block 4g + e/2; groups 2 and 3 hold zeros
+        const unsigned mw = g >= 2 ? 0u
+                            : g == 0 ? e[2] & 0x3F3F3F3Fu
+                                     : ((e[3] >> 4) & 0x0F0F0F0Fu) | ((e[2] >> 2) & 0x30303030u);
+        am[t] = frag(as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04000400u)) - h2(1024.f)),
+                     as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04010401u)) - h2(1024.f)),
+                     as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04020402u)) - h2(1024.f)),
+                     as_u(as_h2(__builtin_amdgcn_perm(0x64646464u, mw, 0x04030403u)) - h2(1024.f)));
+      }
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        const int u = i / NF, f = i % NF;
+        __builtin_amdgcn_sched_barrier(0);
+        if (i + 2 < NI) fetch(i + 2);
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          if (f < 4)
+            cc[u & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                a[t][f], x[i & 3], f == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : cc[u & 1][t], 0, 0, 0);
+          else
+            cm[hb ? u & 1 : 0][t] =
+                __builtin_amdgcn_mfma_f32_16x16x32_f16(am[t], x[i & 3], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (f == 1 && u > 0) scale(u - 1);
+      }
+      scale(CN - 1);
+    }
+  };
+  // this wave's scales of the step whose weights just arrived, in f32, where its own lanes read them back in C layout
+  // (rows 4g + r); the wave's own LDS accesses stay in order, and the compiler fence keeps them so
+  auto store_scales = [&](const Weights& w) {
+#pragma unroll
+    for (int t = 0; t < WN; ++t) {
+      if constexpr (BLK32) {
+        scl[(t * 4 + g) * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));
+      } else if constexpr (TQ2) {
+        scl[t * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));  // the same value from every group
+      } else {  // d from the even groups, dmin from the odd ones
+        scl[t * 32 + (g & 1) * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.e[t][0] >> (16 * (g & 1))));
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  };
+  auto barrier = [&] {  // the staged buffer is published; global loads stay in flight
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+
+  // Step i: the weights of ring slot i % DW, which then loads step i + DW; step i + 1's activations into LDS, whose
+  // registers then load step i + 2's.  (Deeper activation and weight rings measured no faster: what a longer round
+  // hides in latency it costs in cold instructions.)
+  auto step = [&](int i, auto slot) {
+    constexpr int d = decltype(slot)::value;
+    const int s = s0 + i;
+    const Weights w = wring[d % DW];
+    load_w(wring[d % DW], s + DW);
+    store_scales(w);
+    stage(xraw, s + 1);  // past the group's last step: zeros into the idle buffer
+    load_x(xraw, s + 2);
+    compute(w, s, std::bool_constant<(d & 1) != 0>{});
+    barrier();
+  };
+  load_x(xraw, s0);
+#pragma unroll
+  for (int v = 0; v < DW; ++v) load_w(wring[v], s0 + v);
+  stage(xraw, s0);
+  load_x(xraw, s0 + 1);
+  barrier();
+  constexpr int U = QK ? 2 : DW;  // steps a loop round: a whole weight ring, both halves of a Q4_K block
+  static_assert(DW <= 2, "a loop round is one or two steps");
+  for (int i = 0; i < per; i += U) {  // a last odd step of a round of two is past the K group's range: zeros
+    step(i, std::integral_constant<int, 0>{});
+    if constexpr (U > 1) step(i + 1, std::integral_constant<int, 1>{});
+  }
+
+  if constexpr (WK > 1) {  // partial sums of the other K groups, added in group order
+    float* red = reinterpret_cast<float*>(lds);
+    if (wk > 0) {
+#pragma unroll
+      for (int t = 0; t < WN; ++t)
+#pragma unroll
+        for (int u = 0; u < CN; ++u)
+          *reinterpret_cast<f32x4*>(red + ((((wk - 1) * RW + wr) * WN + t) * CN + u) * 256 + lane * 4) = acc[t][u];
+    }
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int q = 0; q < WK - 1; ++q)
+#pragma unroll
+      for (int t = 0; t < WN; ++t)
+#pragma unroll
+        for (int u = 0; u < CN; ++u)
+          acc[t][u] += *reinterpret_cast<const f32x4*>(red + (((q * RW + wr) * WN + t) * CN + u) * 256 + lane * 4);
+  }
+  const bool wide = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 15) == 0;  // whole 16-byte groups of rows
+#pragma unroll
+  for (int t = 0; t < WN; ++t)
+#pragma unroll
+    for (int u = 0; u < CN; ++u) {
+      const int row = nw + 16 * t + 4 * g;
+      const int col = m0 + 16 * u + r16;
+      if (col >= M) continue;
+      float* y = Y + static_cast<int64_t>(col) * N + row;
+      if (wide) {
+        if (row < N) *reinterpret_cast<f32x4*>(y) = acc[t][u];
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (row + r < N) y[r] = acc[t][u][r];
+      }
+    }
+}
+
+template <int FMT, int RW, int WN, int CN, int WK, int DW, bool STORE_S>
+hipError_t launch_plan(const GemmCall& c, hipStream_t stream) {
+  // as gemm.hip: with several column groups the row groups are padded to a multiple of 8, so that the column groups of a
+  // row group run on one XCD and share its L2
+  const unsigned gx = (c.n + 16 * WN * RW - 1) / (16 * WN * RW), gy = (c.m + 16 * CN - 1) / (16 * CN);
+  const dim3 grid(gy > 1 ? (gx + 7) / 8 * 8 : gx, gy);
+  constexpr size_t lds = lds_bytes<FMT, RW, WN, CN, WK>();
+  static_assert(lds <= 160 * 1024, "LDS of a workgroup");
+  auto kern = tile_gemm_kernel<FMT, RW, WN, CN, WK, DW, STORE_S>;
+  static std::atomic<unsigned> lds_limit[kMaxDevices];  // this instantiation's allowed dynamic LDS, per device
+  const hipError_t le = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit);
+  if (le != hipSuccess) return le;
+  const Timing tm = timing_slot(gemv_kind(FMT));
+  hipExtLaunchKernelGGL(kern, grid, dim3(64 * RW * WK), lds, stream, tm.start, tm.stop, 0, c.n, c.m, c.k,
+                        c.k / fmt_info(FMT).block, c.sw, c.wq, c.ws, c.xq, c.xd, c.y, c.s);
+  return hipGetLastError();
+}
+
+// The instantiated plans (gemm_tile_plan in abi.hip picks one).  With S, a smaller tile with the same K split runs: its
+// sums run in the same order, so Y is the same bit for bit, and the scattered stores' addresses leave no room for more.
+template <int FMT>
+hipError_t launch_fmt(const GemmCall& c, const TilePlan& p, hipStream_t stream) {
+  if (c.s != nullptr) {
+    switch (p.wk) {
+      case 1: return launch_plan<FMT, 2, 1, 2, 1, 1, true>(c, stream);
+      case 2: return launch_plan<FMT, 2, 1, 2, 2, 1, true>(c, stream);
+      case 4: return launch_plan<FMT, 1, 1, 1, 4, 1, true>(c, stream);
+      case 8: return launch_plan<FMT, 1, 1, 1, 8, 1, true>(c, stream);
+      default: return hipErrorInvalidConfiguration;
+    }
+  }
+  // (Weight rings of two steps where they measured faster and their registers fit.)
+#define KOMP_TILE_PLAN(RW, WN, CN, WK, DW) \
+  if (p.rw == RW && p.wn == WN && p.cn == CN && p.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, DW, false>(c, stream);
+  KOMP_TILE_PLAN(1, 1, 1, 8, 1)
+  KOMP_TILE_PLAN(1, 2, 1, 4, 1)
+  KOMP_TILE_PLAN(2, 1, 2, 4, 1)
+  KOMP_TILE_PLAN(2, 1, 4, 4, 1)
+  KOMP_TILE_PLAN(4, 1, 4, 2, 1)
+  if constexpr (FMT == FMT_Q4_K) {
+    KOMP_TILE_PLAN(4, 1, 8, 2, 1)
+    KOMP_TILE_PLAN(4, 2, 4, 1, 2)
+    KOMP_TILE_PLAN(8, 1, 8, 1, 1)
+  } else {
+    KOMP_TILE_PLAN(4, 2, 4, 1, 1)
+    KOMP_TILE_PLAN(4, 2, 8, 1, (FMT == FMT_Q4_0 || FMT == FMT_IQ4_NL ? 2 : 1))
+    KOMP_TILE_PLAN(4, 2, 8, 2, 1)
+  }
+#undef KOMP_TILE_PLAN
+  return hipErrorInvalidConfiguration;
+}
+
+}  // namespace gemm_tile
+}  // namespace komp

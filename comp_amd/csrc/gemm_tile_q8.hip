@@ -1,0 +1,10 @@
+// The tiled matrix-core GEMM's Q8_0 instantiations (gemm_tile.h).
+#include "gemm_tile.h"
+
+namespace komp {
+
+hipError_t launch_gemm_tile_q8(const GemmCall& c, const TilePlan& p, hipStream_t stream) {
+  return gemm_tile::launch_fmt<FMT_Q8_0>(c, p, stream);
+}
+
+}  // namespace komp

@@ -105,6 +105,14 @@ struct GemmPlan {
   int d;
 };
 
+// Tiled matrix-core GEMM (gemm_tile.h): a workgroup of wk K groups of rw waves covers 16*wn*rw rows and 16*cn columns.
+struct TilePlan {
+  int rw;
+  int wn;
+  int cn;
+  int wk;
+};
+
 struct GemmCall {
   int fmt;
   const uint8_t* wq;
@@ -221,6 +229,11 @@ hipError_t launch_gemv_q4_lean(const GemvCall& c, const GemvPlan& p, hipStream_t
 hipError_t launch_gemv_q4_lean_bytes(const GemvCall& c, const GemvPlan& p, hipStream_t stream);
 size_t gemm_lds_bytes(int fmt, const GemmPlan& p, int k);
 hipError_t launch_gemm(const GemmCall& c, const GemmPlan& p, hipStream_t stream);
+hipError_t launch_gemm_tile_q4(const GemmCall& c, const TilePlan& p, hipStream_t stream);
+hipError_t launch_gemm_tile_iq4(const GemmCall& c, const TilePlan& p, hipStream_t stream);
+hipError_t launch_gemm_tile_q8(const GemmCall& c, const TilePlan& p, hipStream_t stream);
+hipError_t launch_gemm_tile_tq2(const GemmCall& c, const TilePlan& p, hipStream_t stream);
+hipError_t launch_gemm_tile_q4k(const GemmCall& c, const TilePlan& p, hipStream_t stream);
 hipError_t launch_split(int fmt, const uint8_t* w, uint8_t* wq, int16_t* ws, int64_t n, int64_t k, int64_t sw,
                         hipStream_t stream);
 hipError_t launch_quant_q8_0(const float* x, int8_t* xq, float* xd, int64_t nblocks, hipStream_t stream);

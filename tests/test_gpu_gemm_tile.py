@@ -1,0 +1,82 @@
+"""The tiled matrix-core GEMM (komp_*_gemm from 25 columns on): S exact and Y within its bound against the oracle on
+ragged shapes (rows, columns and blocks that leave partial tiles, steps and K groups), and on shapes large enough for
+every plan, where the exact block dots are f64 matrix products of the oracle's decoded weights."""
+
+import numpy as np
+import pytest
+import torch
+
+from comp_amd import host
+from oracle import oracle as O
+from tests.test_gpu_gemm import check, dev
+
+pytestmark = pytest.mark.gpu
+FMTS = ["q4_0", "tq2_0", "q8_0", "iq4_nl", "q4_k"]
+
+# (n, k of 32-value blocks, k of 256-value blocks, m)
+RAGGED = [(1, 672, 1280, 65), (17, 1120, 2304, 70), (129, 1056, 1536, 97), (45, 4192, 2816, 129), (300, 736, 1792, 83)]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("shape", range(len(RAGGED)))
+@pytest.mark.parametrize("extreme", [False, True])
+def test_ragged_shapes_match_oracle(fmt, shape, extreme):
+    n, k32, k256, m = RAGGED[shape]
+    check(fmt, n, k256 if O.FORMATS[fmt]["block"] == 256 else k32, m, 700 + shape, extreme)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_unaligned_scales_and_padded_rows(fmt):
+    k = 1536 if O.FORMATS[fmt]["block"] == 256 else 1120
+    check(fmt, 45, k, 66, 21, ws_offset=8 if fmt == "q4_k" else 1, pad=48)
+
+
+# (n, m) at 1280 or 672 values of K: together they take every plan of gemm_tile_plan on a 256-CU device
+PLANS = [(64, 70), (100, 49), (1100, 49), (1700, 66), (4310, 49), (5500, 60), (5600, 66), (8400, 66), (9940, 300),
+         (6360, 1000), (10960, 300)]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("shape", range(len(PLANS)))
+def test_every_plan(fmt, shape):
+    n, m = PLANS[shape]
+    blk = O.FORMATS[fmt]["block"]
+    k = 1536 if blk == 256 else 736
+    nb = k // blk
+    rng = np.random.default_rng(shape)
+    W = O.weights(fmt, rng, n, k)
+    wq, ws = host.split(fmt, W, n, k)
+    x = O.activations(rng, k, m, block=O.ACT_BLOCK[O.FORMATS[fmt]["act"]])
+    print(f"tile gemm {fmt} n={n} k={k} m={m} plan {host.gemm_plan(fmt, m, n, k)}", flush=True)
+    xq, xd = host.quantize(fmt, dev(x))
+    y, s = host.gemm(fmt, dev(wq), dev(ws), xq, xd, n, k, store_s=True)
+    y_plain, _ = host.gemm(fmt, dev(wq), dev(ws), xq, xd, n, k)
+    assert torch.equal(y, y_plain)
+    v = dev(O.weight_values(fmt, wq, n, k).astype(np.float64)).view(n, nb, blk)
+    q = xq.double().view(m, nb, blk)
+    if fmt == "q4_k":
+        sc, mn = (dev(a.astype(np.float64)) for a in O.q4_k_scales(ws.view(np.uint8).reshape(n, nb, 16)[:, :, 4:]))
+        v = (v.view(n, nb, 8, 32) * sc[..., None]).reshape(n, nb, 256)
+        qs = q.view(m, nb, 8, 32).sum(3)
+        d = dev(O.f16_bits_to_f32(ws.reshape(n, nb, 8)[:, :, 0]).astype(np.float64))
+        dmin = dev(O.f16_bits_to_f32(ws.reshape(n, nb, 8)[:, :, 1]).astype(np.float64))
+    else:
+        d = dev(O.f16_bits_to_f32(ws).astype(np.float64))
+    ref = torch.zeros((m, n), dtype=torch.float64, device="cuda")
+    mag = torch.zeros_like(ref)  # the terms' magnitudes
+    for b in range(nb):
+        dots = q[:, b] @ v[:, b].T.contiguous()  # exact: integers below 2^53
+        scale = xd[:, b, None].double() * d[None, :, b]
+        if fmt == "q4_k":
+            mins = qs[:, b] @ mn[:, b].T.contiguous()
+            assert torch.equal(s[:, :, b, 0].double(), dots) and torch.equal(s[:, :, b, 1].double(), mins)
+            ms = xd[:, b, None].double() * dmin[None, :, b]
+            ref += scale * dots - ms * mins
+            mag += (scale * dots).abs() + (ms * mins).abs()
+        else:
+            assert torch.equal(s[:, :, b].double(), dots)
+            ref += scale * dots
+            mag += (scale * dots).abs()
+    # each term takes at most 4 roundings of its own and nb (q4_k: 2 nb) in the running sum, plus the K groups' sums
+    assert bool(((y.double() - ref).abs() <= (2 * nb + 16) * 2.0**-24 * mag).all())
+    assert float((y.double() - ref).norm() / ref.norm()) <= 1e-6
