@@ -399,61 +399,66 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
   return gemm_lds_bytes(fmt, q, static_cast<int>(k)) <= kLdsMax;
 }
 
-// The tiled GEMM (gemm_tile.h) takes the larger batches, where its staged activations pay.  Measured on MI355X against
-// gemm.hip's kernel (graph replays) over 9 shapes (127 x 4096 to 28672 x 4096) and 12 column counts: from 25 columns on
-// it is 1.9 times as fast in the geometric mean, at best 5.3 times (Q4_0 14336 x 4096 at 512 columns 385 -> 119 us, TQ2_0
-// 6912 x 2560 at 2048 columns 326 -> 67, Q4_K 4096 x 14336 at 1001 columns 561 -> 215); up to 24 (Q4_K: 48) columns
-// gemm.hip's kernel, which unpacks fewer activations and splits K 8 ways, is as fast or faster (Q4_K 4096 x 14336 at 32
-// columns 23.6 against 27.9 us), and so it is on rows of at most 4 K steps, which are over before the tile's staging
-// pays.
+// The tiled GEMM (gemm_tile.h) takes every batch whose rows are long enough.  Measured on MI355X against gemm.hip's kernel
+// (graph replays, cold weights) over 10 shapes (127 x 4096 to 28672 x 4096) and 14 column counts from 4 to 2048 it is
+// faster at nearly all of them: Q4_0 28672 x 4096 at 16 columns 30.8 -> 20.1 us, 14336 x 4096 at 64 columns 35 -> 24, at
+// 512 columns 385 -> 116, Q8_0 14336 x 4096 at 16 columns 24.3 -> 14.1, TQ2_0 6912 x 2560 at 8 columns 6.3 -> 4.7, at 2048
+// columns 326 -> 61, Q4_K 4096 x 14336 at 1001 columns 561 -> 181.  gemm.hip's kernel keeps
+//   rows of at most 4 K steps, which are over before the tile's staging pays;
+//   Q4_K's few columns, whose scale products the tile multiplies into the weights once per column group: up to 8 columns
+//     (4096 x 14336 12.8 us against 15.3, 28672 x 4096 at 4 columns 22.9 against 24.8), up to 16 over at most 2 row tiles
+//     a CU (2560 x 6912 at 16 columns 8.8 against 9.4); up to 32 where two column groups are just past a workgroup a CU
+//     (2560 x 6912 at 24 columns 11.3 against 13.7); and 49-64 columns over at most 3 row tiles a CU (4096 x 14336 40 us
+//     in one group of 64 columns and in the tile's narrower ones).
 //
 // The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
-// launch has 3 us besides.  The constants are a least-squares fit over those shapes (estimates within 2-6% in the
-// median), and the plan they pick is within 1.2% of the fastest one in the geometric mean (at worst 16%).
+// launch has 3 us besides.  The constants are a least-squares fit over those shapes; the plan they pick is within 1% of
+// the fastest one in the geometric mean.
 struct TileCost {
   TilePlan p;
-  int slots;
-  float ab[3][2];  // (a, b): Q4_0 and IQ4_NL, TQ2_0, Q8_0
+  struct {
+    int slots;  // 0: the format has no such plan
+    float a, b;
+  } f[4];  // Q4_0 and IQ4_NL, TQ2_0, Q8_0, Q4_K
 };
 constexpr TileCost kTileCosts[] = {
-    {{1, 1, 1, 8}, 2, {{0.f, 0.80f}, {0.f, 0.82f}, {0.f, 0.99f}}},
-    {{1, 2, 1, 4}, 4, {{0.12f, 0.57f}, {0.01f, 0.59f}, {0.05f, 0.81f}}},
-    {{2, 1, 2, 4}, 2, {{0.23f, 0.75f}, {0.f, 0.82f}, {0.03f, 1.02f}}},
-    {{2, 1, 4, 4}, 1, {{0.f, 1.71f}, {0.f, 1.59f}, {0.f, 2.01f}}},
-    {{4, 1, 4, 2}, 2, {{0.28f, 0.96f}, {0.10f, 0.90f}, {0.28f, 1.10f}}},
-    {{4, 2, 4, 1}, 3, {{0.61f, 0.71f}, {0.26f, 0.70f}, {0.69f, 0.83f}}},
-    {{4, 2, 8, 1}, 2, {{1.15f, 1.14f}, {0.31f, 1.33f}, {1.31f, 1.30f}}},
-    {{4, 2, 8, 2}, 1, {{0.f, 3.91f}, {0.f, 2.95f}, {0.f, 4.38f}}},
-};
-// Q4_K's waves also hold a block's first half of every output, so its large tiles are half as tall.
-constexpr TileCost kTileCostsQ4K[] = {
-    {{1, 1, 1, 8}, 2, {{0.24f, 0.73f}}}, {{1, 2, 1, 4}, 4, {{0.41f, 0.55f}}}, {{2, 1, 2, 4}, 2, {{0.44f, 0.69f}}},
-    {{2, 1, 4, 4}, 1, {{0.f, 1.77f}}},   {{4, 1, 4, 2}, 1, {{0.f, 1.36f}}},   {{4, 1, 8, 2}, 1, {{0.f, 2.09f}}},
-    {{4, 2, 4, 1}, 2, {{0.41f, 0.73f}}}, {{8, 1, 8, 1}, 1, {{0.f, 1.75f}}},
+    {{1, 1, 1, 8}, {{2, 0.f, 0.58f}, {2, 0.f, 0.74f}, {2, 0.f, 0.65f}, {1, 0.f, 0.99f}}},
+    {{1, 2, 1, 8}, {{2, 0.f, 0.87f}, {1, 0.f, 1.22f}, {2, 0.f, 1.06f}, {1, 0.f, 1.37f}}},
+    {{1, 2, 1, 4}, {{4, 0.11f, 0.41f}, {3, 0.08f, 0.45f}, {4, 0.04f, 0.53f}, {3, 0.30f, 0.47f}}},
+    {{2, 1, 2, 4}, {{2, 0.13f, 0.80f}, {2, 0.f, 0.78f}, {1, 0.f, 0.99f}, {1, 0.f, 1.04f}}},
+    {{2, 2, 2, 4}, {{1, 0.f, 1.60f}, {1, 0.f, 1.41f}, {1, 0.f, 1.83f}, {1, 0.f, 1.59f}}},
+    {{2, 1, 4, 4}, {{1, 0.f, 1.82f}, {1, 0.f, 1.62f}, {1, 0.f, 1.88f}, {1, 0.f, 1.61f}}},
+    {{4, 1, 4, 2}, {{2, 0.07f, 1.11f}, {2, 0.f, 0.97f}, {1, 0.f, 1.28f}, {1, 0.f, 1.19f}}},
+    {{4, 1, 8, 2}, {{1, 0.f, 2.39f}, {1, 0.f, 1.84f}, {1, 0.f, 2.42f}, {1, 0.f, 1.92f}}},
+    {{4, 2, 4, 1}, {{3, 0.58f, 0.73f}, {2, 0.36f, 0.62f}, {3, 0.54f, 0.85f}, {2, 0.52f, 0.65f}}},
+    {{4, 2, 8, 1}, {{2, 1.14f, 1.22f}, {2, 0.61f, 1.08f}, {1, 0.f, 2.29f}, {0, 0.f, 0.f}}},
+    {{4, 2, 8, 2}, {{1, 0.f, 3.59f}, {1, 0.f, 2.84f}, {1, 0.f, 3.77f}, {0, 0.f, 0.f}}},
+    {{8, 1, 8, 1}, {{1, 0.f, 1.92f}, {1, 0.f, 1.44f}, {1, 0.f, 2.03f}, {1, 0.f, 1.63f}}},
 };
 
-// False when the call stays on gemm.hip's kernel: few columns, short rows, or past the tile's 32-bit buffer offsets
-// (128 rows of SW bytes, 128 columns of K) or the grid's column groups.
+// False when the call stays on gemm.hip's kernel: by the rules above, or past the tile's 32-bit buffer offsets (128 rows
+// of SW bytes, 128 columns of K) or the grid's column groups.
 bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePlan* p) {
   const int64_t nblk = k / fmt_info(fmt).block;
   const int64_t steps = fmt == FMT_Q4_K ? 2 * nblk : fmt == FMT_TQ2_0 ? nblk : (nblk + 3) / 4;
-  if (m <= (fmt == FMT_Q4_K ? 48 : 24) || steps <= 4 || n < 1) return false;
-  // Q4_K's 49-64 columns over at most 3 row tiles a CU: 4096 x 14336 40 us here and there, 6912 x 2560 17.5 -> 14.1 but
-  // 4096 x 4096 15.1 either way; over more, 14336 x 4096 45.1 -> 28.5 us, 28672 x 4096 89 -> 42
-  if (fmt == FMT_Q4_K && m <= 64 && n <= 48 * static_cast<int64_t>(device_cus())) return false;
-  if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
-  const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : 0;
   const int64_t cus = device_cus();
+  if (steps <= 4 || n < 1) return false;
+  if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
+  if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus) || (m <= 32 && n > 8 * cus && n <= 12 * cus) ||
+                          (m > 48 && m <= 64 && n <= 48 * cus)))
+    return false;
+  const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : fmt == FMT_Q4_K ? 3 : 0;
   double best = -1;
-  for (const TileCost& t : fmt == FMT_Q4_K ? kTileCostsQ4K : kTileCosts) {
+  for (const TileCost& t : kTileCosts) {
+    const auto& f = t.f[row];
     const int64_t groups = (m + 16 * t.p.cn - 1) / (16 * t.p.cn);
-    if (groups > 65535) continue;
+    if (f.slots == 0 || groups > 65535) continue;
     const int64_t wgs = (n + 16 * t.p.wn * t.p.rw - 1) / (16 * t.p.wn * t.p.rw) * groups;
     const int64_t load = (wgs + cus - 1) / cus;  // workgroups on the fullest CU
     const int64_t per = fmt == FMT_Q4_K ? 2 * ((nblk + t.p.wk - 1) / t.p.wk) : (steps + t.p.wk - 1) / t.p.wk;
-    const double rounds = load > t.slots ? static_cast<double>(load) / t.slots : 1.0;
-    const double us = per * (t.ab[row][0] * rounds + t.ab[row][1] * static_cast<double>(load));
+    const double rounds = load > f.slots ? static_cast<double>(load) / f.slots : 1.0;
+    const double us = per * (f.a * rounds + f.b * static_cast<double>(load));
     if (best < 0 || us < best) {
       best = us;
       *p = t.p;

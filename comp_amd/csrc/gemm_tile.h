@@ -15,18 +15,28 @@
 //     higher rate).
 //   TQ2_0's 256-value blocks stay on v_mfma_i32_16x16x64_i8 (twice the f16 rate; the scaling is 1/8 as often).
 //
+//   With one column tile (up to 16 columns) the 32-value blocks go through v_mfma_i32_16x16x32_i8: there the way of the
+//     weights and activations to f16 costs more than the converted results.
+//
 // Tile.  A workgroup of WK x RW waves owns 16*WN*RW weight rows x 16*CN columns.  The waves of a K group split its rows
-// (each unpacks its own weights from registers, no wave twice) and share its staged activations; the WK groups take
-// contiguous K ranges and add their partial sums at the end in group order.  A K step is 64 bytes of each weight row
-// (Q8_0: 128): 128 values (TQ2_0: 256).  Two LDS buffers: during step i every thread unpacks its share of step i+1's
-// activations (loaded a step earlier) into the other buffer, so one barrier a step suffices and every global load has a
-// whole step to arrive.
+// (each unpacks its own weights, no wave twice) and share its staged activations; the WK groups take contiguous K ranges
+// and add their partial sums at the end in group order.  A K step is 64 bytes of each weight row (Q8_0: 128): 128 values
+// (TQ2_0: 256).  Two LDS buffers: during step i every thread unpacks its share of step i+1's activations (loaded a step
+// earlier) into the other buffer, so one barrier a step suffices and every global load has a whole step to arrive.  A K
+// group of one wave (RW 1) reads back its own staging only and has no barrier at all.
+//
+// Loads.  Four consecutive lanes read 64 consecutive bytes, and the wave's own LDS turns the weights into operand order.
+// Loaded in operand order (16 rows apart lane by lane) a load held the address unit 49 cycles instead of 16, half of
+// the kernel's time at 16 columns: Q4_0 28672 x 4096 24.0 -> 20.1 us, Q8_0 4096 x 14336 16.6 -> 13.3.
 //
 // LDS.  Operand unit (piece, group g) of a column is 16 bytes; units lie [piece][g][column ^ g], so a fragment read
 // covers 256 contiguous, aligned bytes per 16 lanes (a permutation of 4 columns within it).  The staging writes several
 // pieces (TQ2_0: and groups) of one column at a time: a pad of 64 bytes after each piece and the column's low bits
 // crossed with g put those on different banks.  (Padding every unit row by 16 bytes instead left the reads with 42% of
 // their LDS cycles in conflicts.)
+//
+// What it reaches: IQ4_NL 14336 x 4096 at 2048 columns issues VALU instructions 81% of the time (about 890 a wave and
+// step, 512 of them the scaling), matrix instructions 23%; TQ2_0 6912 x 2560 at 2048 columns 1.19 POP/s.
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -40,6 +50,7 @@ namespace komp {
 namespace gemm_tile {
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
@@ -49,19 +60,6 @@ constexpr unsigned kOob = 0x7FFFFFF0u;  // an offset past every descriptor's ran
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void* base, int64_t bytes) {
   const int n = static_cast<int>(bytes <= 0 ? 0 : (bytes < 0x7FFFFFF0 ? bytes : 0x7FFFFFF0));
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, n, kRsrcWord3);
-}
-
-// 4x4 dword transpose across the four 16-lane rows of a wave: on entry row g of v[q] holds element (q, g), on exit row
-// g of t[j] holds element (g, j).
-__device__ __forceinline__ void transpose4(const u32x4& v, unsigned (&t)[4]) {
-  const auto a = __builtin_amdgcn_permlane32_swap(v[0], v[2], false, false);
-  const auto b = __builtin_amdgcn_permlane32_swap(v[1], v[3], false, false);
-  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
-  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
-  t[0] = c[0];
-  t[1] = c[1];
-  t[2] = d[0];
-  t[3] = d[1];
 }
 
 __device__ __forceinline__ f16x2 as_h2(unsigned v) { return __builtin_bit_cast(f16x2, v); }
@@ -81,27 +79,34 @@ __device__ __forceinline__ f16x8 frag(unsigned a, unsigned b, unsigned c, unsign
 
 // LDS bytes of one K group's part: two activation buffers, two d_x buffers and (Q4_K) two buffers of 16-value sums; and
 // of one wave's scales.
+constexpr bool blk32(int fmt) { return fmt == FMT_Q4_0 || fmt == FMT_IQ4_NL || fmt == FMT_Q8_0; }
+
 template <int FMT, int CN>
 struct Lds {
-  static constexpr int kRow = 16 * CN * 16;                // a unit row: 16 bytes a column
+  static constexpr int kUnit = blk32(FMT) && CN == 1 ? 8 : 16;  // int8 operands, or f16 ones (TQ2_0: 16 int8)
+  static constexpr int kRow = 16 * CN * kUnit;             // a unit row: a unit a column
   static constexpr int kPiece = 4 * kRow + 64;             // the four groups' rows of a piece, and the pad
   static constexpr int kBuf = 4 * kPiece;
   static constexpr int kDx = 16 * CN * (FMT == FMT_TQ2_0 || FMT == FMT_Q4_K ? 1 : 4) * 4;
   static constexpr int kSums = FMT == FMT_Q4_K ? 2 * kRow : 0;
   static constexpr int kGroup = 2 * (kBuf + kDx + kSums);
-  static constexpr int scales(int wn) {  // f32 per wave: 4 blocks of 16 rows a tile; TQ2_0 one; Q4_K d and dmin
-    return wn * 16 * (FMT == FMT_TQ2_0 ? 1 : FMT == FMT_Q4_K ? 2 : 4) * 4;
+  // one wave's part: 64 weight bytes of each row, f32 scales (4 blocks of 16 rows a tile; TQ2_0 one; Q4_K d and dmin)
+  // and (Q4_K) the rows' 16 scale-plane bytes
+  static constexpr int weights(int wn) { return wn * 1024; }
+  static constexpr int scales(int wn) {
+    return wn * 16 * (FMT == FMT_TQ2_0 ? 1 : FMT == FMT_Q4_K ? 2 : 4) * 4 + (FMT == FMT_Q4_K ? wn * 256 : 0);
   }
+  static constexpr int wave(int wn) { return weights(wn) + scales(wn); }
 };
 
 template <int FMT, int RW, int WN, int CN, int WK>
 constexpr size_t lds_bytes() {
-  const size_t stage = static_cast<size_t>(WK) * Lds<FMT, CN>::kGroup + WK * RW * Lds<FMT, CN>::scales(WN);
+  const size_t stage = static_cast<size_t>(WK) * Lds<FMT, CN>::kGroup + WK * RW * Lds<FMT, CN>::wave(WN);
   const size_t red = static_cast<size_t>(WK - 1) * RW * WN * CN * 4 * 64 * 4;
   return stage > red ? stage : red;
 }
 
-template <int FMT, int RW, int WN, int CN, int WK, int DW, bool STORE_S>
+template <int FMT, int RW, int WN, int CN, int WK, bool STORE_S>
 __global__ void __launch_bounds__(64 * RW * WK, RW * WK == 4 ? 2 : 1)
 tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __restrict__ WQ,
                  const int16_t* __restrict__ WS, const int8_t* __restrict__ XQ, const float* __restrict__ XD,
@@ -111,14 +116,18 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   constexpr bool BLK32 = NIB4 || Q8;
   constexpr bool TQ2 = FMT == FMT_TQ2_0;
   constexpr bool QK = FMT == FMT_Q4_K;
+  constexpr bool I8 = BLK32 && CN == 1;
   using L = Lds<FMT, CN>;
   constexpr int T = 64 * RW;          // threads of a K group
   constexpr int COLS = 16 * CN;
   constexpr int WGR = 16 * WN * RW;   // rows of the workgroup
   constexpr int WV = Q8 ? 2 : 1;      // 16-byte weight loads per row tile and step
   constexpr int XB = TQ2 ? 256 : 128;  // activation bytes per column and step
-  constexpr int BI = TQ2 ? COLS * 16 / T : COLS * 4 / T;  // staging items a thread: 16 bytes (TQ2_0) or 32
-  static_assert(BI * T == (TQ2 ? COLS * 16 : COLS * 4), "the threads split the staged columns evenly");
+  constexpr bool F16 = !TQ2 && !I8;    // activations staged as f16
+  constexpr int XV = F16 ? 2 : 1;      // 16-byte loads an item
+  constexpr int PC = XB / 16 / XV;     // staging items of a column and step: 16 bytes (F16: a block's 32)
+  constexpr int BI = COLS * PC / T;    // staging items a thread
+  static_assert(BI * T == COLS * PC, "the threads split the staged columns evenly");
   extern __shared__ __align__(16) unsigned char lds[];
   // kBias in a VGPR, so that masking a nibble pair and putting the bias on is one v_and_or_b32 (which takes one literal)
   unsigned bias;
@@ -144,7 +153,8 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   unsigned char* const gl = lds + wk * L::kGroup;
   unsigned char* const dxl = gl + 2 * L::kBuf;
   unsigned char* const suml = dxl + 2 * L::kDx;
-  float* const scl = reinterpret_cast<float*>(lds + WK * L::kGroup + wave * L::scales(WN));
+  unsigned char* const wl = lds + WK * L::kGroup + wave * L::wave(WN);
+  float* const scl = reinterpret_cast<float*>(wl + L::weights(WN));
 
   const auto wq = rsrc(WQ + nw * SW, rows * SW);
   const auto ws = rsrc(WS + static_cast<int64_t>(nw) * nblk * (QK ? 8 : 1),
@@ -153,33 +163,41 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   const auto xd = rsrc(XD + static_cast<int64_t>(m0) * nblk, static_cast<int64_t>(cols) * nblk * 4);
 
   // ---- global loads, a step's worth each ----
+  // Four consecutive lanes read consecutive addresses in every load (a row's 64 weight bytes, its 4 scales, 4 pieces of
+  // a column): the address unit takes such a quad at once, and lanes that jump from row to row one by one (Q4_0
+  // 28672 x 4096 at 16 columns, loads in the operands' lane order: 49 cycles a load, half of the kernel's time).
+  const int lr = lane >> 2, lp = lane & 3;  // the lane's row and piece of a tile's load
   unsigned va[WN], vs[WN];
 #pragma unroll
   for (int t = 0; t < WN; ++t) {
-    va[t] = static_cast<unsigned>((16 * t + r16) * SW + 16 * g);
-    vs[t] = static_cast<unsigned>((16 * t + r16) * nblk * (QK ? 16 : 2));
+    va[t] = static_cast<unsigned>((16 * t + lr) * SW + 16 * lp);
+    vs[t] = TQ2 ? static_cast<unsigned>((16 * t + r16) * nblk * 2) : static_cast<unsigned>((16 * t + lr) * nblk * (QK ? 16 : 2));
   }
   unsigned vx[BI], lx[BI];  // an item's source offset and its LDS offset
 #pragma unroll
   for (int i = 0; i < BI; ++i) {
     const int idx = i * T + tid;
-    if constexpr (TQ2) {  // 16 bytes q of a column: half q/8, crumb (q%8)/2, 16-byte half q%2 of the 32
-      const int q = idx & 15, c = idx >> 4;
-      vx[i] = static_cast<unsigned>(c * K + 16 * q);
-      const int j = (q & 7) >> 1, gq = (q >> 3) * 2 + (q & 1);
+    const int p = idx % PC, c = idx / PC;
+    vx[i] = static_cast<unsigned>(c * K + 16 * XV * p);
+    if constexpr (TQ2) {  // half p/8, crumb (p%8)/2, 16-byte half p%2 of the 32
+      const int j = (p & 7) >> 1, gq = (p >> 3) * 2 + (p & 1);
       lx[i] = static_cast<unsigned>(j * L::kPiece + gq * L::kRow + 16 * (c ^ gq));
-    } else {  // block j of a column
-      const int j = idx & 3, c = idx >> 2;
-      vx[i] = static_cast<unsigned>(c * K + 32 * j);
-      lx[i] = static_cast<unsigned>(j * L::kPiece + 16 * c);
+    } else if constexpr (F16) {  // block p: its unit of every group
+      lx[i] = static_cast<unsigned>(p * L::kPiece + L::kUnit * c);
+    } else {  // half p%2 of block p/2: half of the block's unit of every group
+      lx[i] = static_cast<unsigned>((p >> 1) * L::kPiece + L::kUnit * c + (p & 1) * (L::kUnit / 2));
     }
   }
+  // A tile's weights in the wave's LDS: row lr at 64 lr, its 16-byte pieces in the order p ^ f, f = -(row / 4) mod 4, so
+  // that a dword of each row, or a piece of each row, is read from all banks
+  const unsigned lw = static_cast<unsigned>(64 * lr + 16 * (lp ^ (-(lr >> 2) & 3)));
+  const unsigned fr = static_cast<unsigned>(-(r16 >> 2) & 3);
   struct Weights {  // one step's weights and scales of the wave's rows
     u32x4 a[WN][WV];
-    u32x4 e[QK ? WN : 1];        // Q4_K: the block's 16 scale-plane bytes
+    unsigned e[QK ? WN : 1];     // Q4_K: dword lp of the block's 16 scale-plane bytes
     unsigned short h[QK ? 1 : WN];
   };
-  Weights wring[DW];
+  Weights wraw;
   auto load_w = [&](Weights& w, int s) {
     const unsigned off = s < s1 ? 64u * WV * s : kOob;
 #pragma unroll
@@ -188,16 +206,16 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       for (int v = 0; v < WV; ++v)
         w.a[t][v] = __builtin_amdgcn_raw_buffer_load_b128(wq, va[t] + off + 64 * v, 0, 0);
       if constexpr (QK)
-        w.e[t] = __builtin_amdgcn_raw_buffer_load_b128(ws, vs[t] + (s < s1 ? 16u * (s >> 1) : kOob), 0, 0);
+        w.e[t] = __builtin_amdgcn_raw_buffer_load_b32(ws, vs[t] + (s < s1 ? 16u * (s >> 1) + 4u * lp : kOob), 0, 0);
       else if constexpr (TQ2)
-        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 ? 2u * s : kOob), 0, 0);
+        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 && g == 0 ? 2u * s : kOob), 0, 0);
       else  // a block past K has scale zero
-        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 && 4 * s + g < nblk ? 8u * s + 2u * g : kOob),
+        w.h[t] = __builtin_amdgcn_raw_buffer_load_b16(ws, vs[t] + (s < s1 && 4 * s + lp < nblk ? 8u * s + 2u * lp : kOob),
                                                        0, 0);
     }
   };
-  constexpr int XV = TQ2 ? 1 : 2;
-  constexpr int DI = BLK32 ? BI : (COLS + T - 1) / T;
+  constexpr int DN = BLK32 ? COLS * 4 : COLS;  // d_x of a step: [column][block]
+  constexpr int DI = (DN + T - 1) / T;
   struct Acts {  // one step's activations, this thread's share
     u32x4 x[BI][XV];
     float d[DI];
@@ -208,16 +226,16 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int v = 0; v < XV; ++v)
-        a.x[i][v] = __builtin_amdgcn_raw_buffer_load_b128(xq, vx[i] + off + 16 * v, 0, 0);
+      for (int v = 0; v < XV; ++v) a.x[i][v] = __builtin_amdgcn_raw_buffer_load_b128(xq, vx[i] + off + 16 * v, 0, 0);
 #pragma unroll
     for (int i = 0; i < DI; ++i) {
       const int idx = i * T + tid;
       unsigned o;
       if constexpr (BLK32)
-        o = s < s1 && 4 * s + (idx & 3) < nblk ? static_cast<unsigned>((idx >> 2) * nblk + 4 * s + (idx & 3)) * 4u : kOob;
+        o = s < s1 && idx < DN && 4 * s + (idx & 3) < nblk
+                ? static_cast<unsigned>((idx >> 2) * nblk + 4 * s + (idx & 3)) * 4u : kOob;  // fmt: skip
       else
-        o = s < s1 && idx < COLS ? static_cast<unsigned>(idx * nblk + (QK ? s >> 1 : s)) * 4u : kOob;
+        o = s < s1 && idx < DN ? static_cast<unsigned>(idx * nblk + (QK ? s >> 1 : s)) * 4u : kOob;
       a.d[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xd, o, 0, 0));
     }
   };
@@ -231,18 +249,22 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
         *reinterpret_cast<u32x4*>(b + lx[i]) = a.x[i][0];
       } else {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {  // group q: values 4q..4q+3 and 16+4q..16+4q+3
-          u32x4 u;
-          unsigned e, o;
-          bytes_to_f16(a.x[i][0][q], e, o);
-          u[0] = e;
-          u[1] = o;
-          bytes_to_f16(a.x[i][1][q], e, o);
-          u[2] = e;
-          u[3] = o;
-          *reinterpret_cast<u32x4*>(b + (lx[i] ^ (16 * q)) + q * L::kRow) = u;
+        for (int q = 0; q < 4; ++q) {
+          if constexpr (F16) {  // group q: values 4q..4q+3 and 16+4q..16+4q+3
+            u32x4 u;
+            unsigned e, o;
+            bytes_to_f16(a.x[i][0][q], e, o);
+            u[0] = e;
+            u[1] = o;
+            bytes_to_f16(a.x[i][1][q], e, o);
+            u[2] = e;
+            u[3] = o;
+            *reinterpret_cast<u32x4*>(b + (lx[i] ^ (16 * q)) + q * L::kRow) = u;
+          } else {  // dword q of the piece: group q's half of the block's unit
+            *reinterpret_cast<unsigned*>(b + lx[i] + q * L::kRow) = a.x[i][0][q];
+          }
         }
-        if constexpr (QK) {  // the item's two 16-value sums (at most 16 * 128: exact in f16)
+        if constexpr (QK) {  // the block's two 16-value sums (at most 16 * 128: exact in f16)
           const int idx = i * T + tid;
           int lo = 0, hi = 0;
 #pragma unroll
@@ -251,15 +273,15 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
             hi = __builtin_amdgcn_sdot4(static_cast<int>(a.x[i][1][q]), 0x01010101, hi, false);
           }
           const f16x2 p = {static_cast<_Float16>(static_cast<float>(lo)), static_cast<_Float16>(static_cast<float>(hi))};
-          *reinterpret_cast<unsigned*>(suml + (((s - s0) >> 1) & 1) * L::kSums + (s & 1) * L::kRow + 16 * (idx >> 2) +
-                                       4 * (idx & 3)) = as_u(p);
+          *reinterpret_cast<unsigned*>(suml + (((s - s0) >> 1) & 1) * L::kSums + (s & 1) * L::kRow + 16 * (idx / PC) +
+                                       4 * (idx % PC)) = as_u(p);
         }
       }
     }
 #pragma unroll
     for (int i = 0; i < DI; ++i) {
       const int idx = i * T + tid;
-      if (BLK32 || DI * T == COLS || idx < COLS) dxb[idx] = a.d[i];  // BLK32: [column][block of the step]
+      if (DI * T == DN || idx < DN) dxb[idx] = a.d[i];
     }
   };
 
@@ -289,16 +311,61 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   // that order (left alone, the compiler scales each result right behind its matrix instruction and waits for it), and
   // the empty asm statements pin each sum's update to its place (otherwise it may be moved down to the sum's next use, a
   // step later, with every result of the step kept live: 1000 bytes a lane of spills).
-  auto compute = [&](const Weights& w, int s, auto odd) {
-    const unsigned char* const b = gl + ((s - s0) & 1) * L::kBuf + (r16 ^ g) * 16 + g * L::kRow;
+  // wf[t][v]: a tile's weights in operand order.  TQ2_0: the lane's 16 bytes (row r16, piece g); else dword g of the
+  // row's four 16-byte pieces (nibble formats: of 4 blocks, Q8_0: of 4 half blocks)
+  auto compute = [&](const u32x4 (&wf)[WN][WV], int s, auto odd) {
+    const unsigned char* const b = gl + ((s - s0) & 1) * L::kBuf + (I8 ? r16 * 8 : (r16 ^ g) * 16) + g * L::kRow;
     const unsigned char* const dxp = dxl + ((s - s0) & 1) * L::kDx;
-    if constexpr (BLK32) {
+    if constexpr (I8) {
+      // one column tile: the nibbles' way to f16 would cost more than the converted results save (Q4_0 9 instructions a
+      // tile and block against 3 and 4 conversions), and so would the activations'
+      long x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const long*>(b + j * L::kPiece);
+      const f32x4 dx = *reinterpret_cast<const f32x4*>(dxp + r16 * 16);
+      i32x4 corr[4], cc[2][WN];
+      f32x4 dw[2][WN];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        corr[j] = i32x4{0, 0, 0, 0};
+        if constexpr (FMT == FMT_Q4_0)  // the nibbles go in unsigned: start at -8 times the block's activation sum
+          corr[j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(static_cast<long>(0xF8F8F8F8F8F8F8F8ull), x[j], corr[j], 0, 0, 0);
+      }
+      auto scale = [&](int j) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          f32x4 cf;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) cf[r] = static_cast<float>(cc[j & 1][t][r]);
+          if (STORE_S && 4 * s + j < nblk && s < s1) store_s(cf, t, 0, 4 * s + j, 1, 0, false);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[t][0][r] = __builtin_fmaf(cf[r] * dw[j & 1][t][r], dx[j], acc[t][0][r]);
+          asm volatile("" : "+v"(acc[t][0]));
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int t = 0; t < WN; ++t) {
+          unsigned lo, hi;
+          if constexpr (FMT == FMT_Q4_0) {
+            lo = wf[t][0][j] & 0x0F0F0F0Fu;
+            hi = (wf[t][0][j] >> 4) & 0x0F0F0F0Fu;
+          } else if constexpr (FMT == FMT_IQ4_NL) {
+            iq4_nl_lut(wf[t][0][j], lo, hi);
+          } else {
+            lo = wf[t][j >> 1][2 * (j & 1)];
+            hi = wf[t][j >> 1][2 * (j & 1) + 1];
+          }
+          dw[j & 1][t] = *reinterpret_cast<const f32x4*>(scl + (t * 4 + j) * 16 + 4 * g);
+          cc[j & 1][t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, u32x2{lo, hi}), x[j], corr[j], 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (j > 0) scale(j - 1);
+      }
+      scale(3);
+    } else if constexpr (BLK32) {
       constexpr int NI = 4 * CN;  // i = j * CN + u: block j of the step, column tile u
-      unsigned ta[WN][WV][4];
-#pragma unroll
-      for (int t = 0; t < WN; ++t)
-#pragma unroll
-        for (int v = 0; v < WV; ++v) transpose4(w.a[t][v], ta[t][v]);
       f16x8 a[2][WN], x[4];
       f32x4 dw[2][WN], cc[2][WN], dx[CN];
       auto fetch = [&](int i) {
@@ -308,7 +375,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
 #pragma unroll
         for (int t = 0; t < WN; ++t) {
           if constexpr (FMT == FMT_Q4_0) {
-            const unsigned p = ta[t][0][j], q = p >> 8;
+            const unsigned p = wf[t][0][j], q = p >> 8;
             a[j & 1][t] =
                 frag(as_u(as_h2((p & 0x000F000Fu) | bias) - h2(1032.f)), as_u(as_h2((q & 0x000F000Fu) | bias) - h2(1032.f)),
                      as_u(__builtin_elementwise_fma(as_h2((p & 0x00F000F0u) | bias), h2(0.0625f), h2(-72.f))),
@@ -316,10 +383,10 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           } else {
             unsigned lo, hi, e0, o0, e1, o1;
             if constexpr (FMT == FMT_IQ4_NL) {
-              iq4_nl_lut(ta[t][0][j], lo, hi);
+              iq4_nl_lut(wf[t][0][j], lo, hi);
             } else {
-              lo = ta[t][j >> 1][2 * (j & 1)];
-              hi = ta[t][j >> 1][2 * (j & 1) + 1];
+              lo = wf[t][j >> 1][2 * (j & 1)];
+              hi = wf[t][j >> 1][2 * (j & 1) + 1];
             }
             bytes_to_f16(lo, e0, o0);
             bytes_to_f16(hi, e1, o1);
@@ -387,8 +454,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
         for (int v = 0; v < 4; ++v)
 #pragma unroll
           for (int d = 0; d < 4; ++d)  // crumbs 0..3 -> -1, 0, 1, 2 (a byte table lookup)
-            a[t][v][d] = static_cast<int>(
-                __builtin_amdgcn_perm(0, 0x020100FFu, (w.a[t][0][d] >> (2 * v)) & 0x03030303u));
+            a[t][v][d] = static_cast<int>(__builtin_amdgcn_perm(0, 0x020100FFu, (wf[t][0][d] >> (2 * v)) & 0x03030303u));
       }
 #pragma unroll
       for (int u = 0; u < CN; ++u) {
@@ -450,11 +516,9 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
 #pragma unroll
       for (int t = 0; t < WN; ++t) {
-        unsigned ta[4];
-        transpose4(w.a[t][0], ta);
         if constexpr (hb) dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 4 * g);
         if constexpr (hb) dm[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 16 + 4 * g);
-        const u32x4 e = w.e[t];
+        const u32x4 e = *reinterpret_cast<const u32x4*>(scl + WN * 32 + t * 64 + r16 * 4);
         const unsigned sc = hb ? (e[3] & 0x0F0F0F0Fu) | ((e[1] >> 2) & 0x30303030u) : e[1] & 0x3F3F3F3Fu;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -464,7 +528,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           const f16x2 m = (i & 1) ? f * h2(0.0625f) : f;
           const f16x2 k = f * h2((i & 1) ? -64.f : -1024.f);
           const unsigned mask = (i & 1) ? 0x00F000F0u : 0x000F000Fu;
-          const unsigned p0 = ta[2 * (i >> 1)], p1 = ta[2 * (i >> 1) + 1];
+          const unsigned p0 = wf[t][0][2 * (i >> 1)], p1 = wf[t][0][2 * (i >> 1) + 1];
           a[t][i] = frag(as_u(__builtin_elementwise_fma(as_h2((p0 & mask) | bias), m, k)),
                          as_u(__builtin_elementwise_fma(as_h2(((p0 >> 8) & mask) | bias), m, k)),
                          as_u(__builtin_elementwise_fma(as_h2((p1 & mask) | bias), m, k)),
@@ -499,56 +563,79 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       scale(CN - 1);
     }
   };
-  // this wave's scales of the step whose weights just arrived, in f32, where its own lanes read them back in C layout
-  // (rows 4g + r); the wave's own LDS accesses stay in order, and the compiler fence keeps them so
-  auto store_scales = [&](const Weights& w) {
+  // this step's weights and f32 scales through the wave's own LDS, from where its lanes read them back in operand and C
+  // layout (rows 4g + r); the wave's own LDS accesses stay in order, and the compiler fences keep them so
+  auto take_w = [&](const Weights& w, u32x4 (&wf)[WN][WV]) {
 #pragma unroll
     for (int t = 0; t < WN; ++t) {
       if constexpr (BLK32) {
-        scl[(t * 4 + g) * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));
+        scl[(t * 4 + lp) * 16 + lr] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));
       } else if constexpr (TQ2) {
-        scl[t * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));  // the same value from every group
-      } else {  // d from the even groups, dmin from the odd ones
-        scl[t * 32 + (g & 1) * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.e[t][0] >> (16 * (g & 1))));
+        if (g == 0) scl[t * 16 + r16] = f16_bits_to_f32(static_cast<int16_t>(w.h[t]));
+      } else {  // d from the even pieces' lanes, dmin from the odd ones': both in dword 0
+        reinterpret_cast<unsigned*>(scl)[WN * 32 + t * 64 + lane] = w.e[t];
+        const unsigned d0 = static_cast<unsigned>(dpp_i<0x00>(static_cast<int>(w.e[t])));  // quad_perm [0, 0, 0, 0]
+        scl[t * 32 + (lp & 1) * 16 + lr] = f16_bits_to_f32(static_cast<int16_t>(d0 >> (16 * (lp & 1))));
       }
     }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int v = 0; v < WV; ++v) {
+#pragma unroll
+      for (int t = 0; t < WN; ++t) *reinterpret_cast<u32x4*>(wl + t * 1024 + lw) = w.a[t][v];
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+      for (int t = 0; t < WN; ++t) {
+        if constexpr (TQ2) {
+          wf[t][v] = *reinterpret_cast<const u32x4*>(wl + t * 1024 + 64 * r16 + 16 * (g ^ fr));
+        } else {
+#pragma unroll
+          for (unsigned j = 0; j < 4; ++j)
+            wf[t][v][j] = *reinterpret_cast<const unsigned*>(wl + t * 1024 + 64 * r16 + 4 * g + 16 * (j ^ fr));
+        }
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
   };
   auto barrier = [&] {  // the staged buffer is published; global loads stay in flight
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    if constexpr (RW == 1) {  // a wave reads back its own staging only: its LDS accesses stay in order
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    } else {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    }
   };
 
-  // Step i: the weights of ring slot i % DW, which then loads step i + DW; step i + 1's activations into LDS, whose
-  // registers then load step i + 2's.  (Deeper activation and weight rings measured no faster: what a longer round
-  // hides in latency it costs in cold instructions.)
-  auto step = [&](int i, auto slot) {
-    constexpr int d = decltype(slot)::value;
+  // Step i: its weights and step i + 1's activations from the registers into LDS, then the loads of the next ones into the
+  // same registers.  (Deeper rings of loads measured no faster: a longer loop round costs more in cold instructions than
+  // it hides in latency.)
+  auto step = [&](int i, auto odd) {
     const int s = s0 + i;
-    const Weights w = wring[d % DW];
-    load_w(wring[d % DW], s + DW);
-    store_scales(w);
+    u32x4 wf[WN][WV];
+    take_w(wraw, wf);
+    load_w(wraw, s + 1);
     stage(xraw, s + 1);  // past the group's last step: zeros into the idle buffer
     load_x(xraw, s + 2);
-    compute(w, s, std::bool_constant<(d & 1) != 0>{});
+    compute(wf, s, odd);
     barrier();
   };
   load_x(xraw, s0);
-#pragma unroll
-  for (int v = 0; v < DW; ++v) load_w(wring[v], s0 + v);
+  load_w(wraw, s0);
   stage(xraw, s0);
   load_x(xraw, s0 + 1);
   barrier();
-  constexpr int U = QK ? 2 : DW;  // steps a loop round: a whole weight ring, both halves of a Q4_K block
-  static_assert(DW <= 2, "a loop round is one or two steps");
-  for (int i = 0; i < per; i += U) {  // a last odd step of a round of two is past the K group's range: zeros
-    step(i, std::integral_constant<int, 0>{});
-    if constexpr (U > 1) step(i + 1, std::integral_constant<int, 1>{});
+  if constexpr (QK) {  // per is even: s0 + i is the first half of a block
+    for (int i = 0; i < per; i += 2) {
+      step(i, std::false_type{});
+      step(i + 1, std::true_type{});
+    }
+  } else {
+    for (int i = 0; i < per; ++i) step(i, std::false_type{});
   }
 
   if constexpr (WK > 1) {  // partial sums of the other K groups, added in group order
     float* red = reinterpret_cast<float*>(lds);
+    if constexpr (RW == 1) __syncthreads();  // every wave is done with its staging
     if (wk > 0) {
 #pragma unroll
       for (int t = 0; t < WN; ++t)
@@ -585,7 +672,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
     }
 }
 
-template <int FMT, int RW, int WN, int CN, int WK, int DW, bool STORE_S>
+template <int FMT, int RW, int WN, int CN, int WK, bool STORE_S>
 hipError_t launch_plan(const GemmCall& c, hipStream_t stream) {
   // as gemm.hip: with several column groups the row groups are padded to a multiple of 8, so that the column groups of a
   // row group run on one XCD and share its L2
@@ -593,7 +680,7 @@ hipError_t launch_plan(const GemmCall& c, hipStream_t stream) {
   const dim3 grid(gy > 1 ? (gx + 7) / 8 * 8 : gx, gy);
   constexpr size_t lds = lds_bytes<FMT, RW, WN, CN, WK>();
   static_assert(lds <= 160 * 1024, "LDS of a workgroup");
-  auto kern = tile_gemm_kernel<FMT, RW, WN, CN, WK, DW, STORE_S>;
+  auto kern = tile_gemm_kernel<FMT, RW, WN, CN, WK, STORE_S>;
   static std::atomic<unsigned> lds_limit[kMaxDevices];  // this instantiation's allowed dynamic LDS, per device
   const hipError_t le = allow_dynamic_lds(reinterpret_cast<const void*>(kern), lds, lds_limit);
   if (le != hipSuccess) return le;
@@ -609,29 +696,28 @@ template <int FMT>
 hipError_t launch_fmt(const GemmCall& c, const TilePlan& p, hipStream_t stream) {
   if (c.s != nullptr) {
     switch (p.wk) {
-      case 1: return launch_plan<FMT, 2, 1, 2, 1, 1, true>(c, stream);
-      case 2: return launch_plan<FMT, 2, 1, 2, 2, 1, true>(c, stream);
-      case 4: return launch_plan<FMT, 1, 1, 1, 4, 1, true>(c, stream);
-      case 8: return launch_plan<FMT, 1, 1, 1, 8, 1, true>(c, stream);
+      case 1: return launch_plan<FMT, 2, 1, 2, 1, true>(c, stream);
+      case 2: return launch_plan<FMT, 2, 1, 2, 2, true>(c, stream);
+      case 4: return launch_plan<FMT, 1, 1, 1, 4, true>(c, stream);
+      case 8: return launch_plan<FMT, 1, 1, 1, 8, true>(c, stream);
       default: return hipErrorInvalidConfiguration;
     }
   }
-  // (Weight rings of two steps where they measured faster and their registers fit.)
-#define KOMP_TILE_PLAN(RW, WN, CN, WK, DW) \
-  if (p.rw == RW && p.wn == WN && p.cn == CN && p.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, DW, false>(c, stream);
-  KOMP_TILE_PLAN(1, 1, 1, 8, 1)
-  KOMP_TILE_PLAN(1, 2, 1, 4, 1)
-  KOMP_TILE_PLAN(2, 1, 2, 4, 1)
-  KOMP_TILE_PLAN(2, 1, 4, 4, 1)
-  KOMP_TILE_PLAN(4, 1, 4, 2, 1)
-  if constexpr (FMT == FMT_Q4_K) {
-    KOMP_TILE_PLAN(4, 1, 8, 2, 1)
-    KOMP_TILE_PLAN(4, 2, 4, 1, 2)
-    KOMP_TILE_PLAN(8, 1, 8, 1, 1)
-  } else {
-    KOMP_TILE_PLAN(4, 2, 4, 1, 1)
-    KOMP_TILE_PLAN(4, 2, 8, 1, (FMT == FMT_Q4_0 || FMT == FMT_IQ4_NL ? 2 : 1))
-    KOMP_TILE_PLAN(4, 2, 8, 2, 1)
+#define KOMP_TILE_PLAN(RW, WN, CN, WK) \
+  if (p.rw == RW && p.wn == WN && p.cn == CN && p.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, false>(c, stream);
+  KOMP_TILE_PLAN(1, 1, 1, 8)
+  KOMP_TILE_PLAN(1, 2, 1, 8)
+  KOMP_TILE_PLAN(1, 2, 1, 4)
+  KOMP_TILE_PLAN(2, 1, 2, 4)
+  KOMP_TILE_PLAN(2, 2, 2, 4)
+  KOMP_TILE_PLAN(2, 1, 4, 4)
+  KOMP_TILE_PLAN(4, 1, 4, 2)
+  KOMP_TILE_PLAN(4, 1, 8, 2)
+  KOMP_TILE_PLAN(4, 2, 4, 1)
+  KOMP_TILE_PLAN(8, 1, 8, 1)
+  if constexpr (FMT != FMT_Q4_K) {  // Q4_K's waves also hold a block's first half of every output: too many registers
+    KOMP_TILE_PLAN(4, 2, 8, 1)
+    KOMP_TILE_PLAN(4, 2, 8, 2)
   }
 #undef KOMP_TILE_PLAN
   return hipErrorInvalidConfiguration;

@@ -1,4 +1,4 @@
-"""The tiled matrix-core GEMM (komp_*_gemm from 25 columns on): S exact and Y within its bound against the oracle on
+"""The tiled matrix-core GEMM (komp_*_gemm, rows of more than 4 K steps): S exact and Y within its bound against the oracle on
 ragged shapes (rows, columns and blocks that leave partial tiles, steps and K groups), and on shapes large enough for
 every plan, where the exact block dots are f64 matrix products of the oracle's decoded weights."""
 
@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 FMTS = ["q4_0", "tq2_0", "q8_0", "iq4_nl", "q4_k"]
 
 # (n, k of 32-value blocks, k of 256-value blocks, m)
-RAGGED = [(1, 672, 1280, 65), (17, 1120, 2304, 70), (129, 1056, 1536, 97), (45, 4192, 2816, 129), (300, 736, 1792, 83)]
+RAGGED = [(1, 672, 1280, 5), (33, 4192, 2816, 9), (100, 544, 1280, 16), (70, 1056, 1536, 31), (1, 672, 1280, 65), (17, 1120, 2304, 70), (129, 1056, 1536, 97), (45, 4192, 2816, 129), (300, 736, 1792, 83)]
 
 
 @pytest.mark.parametrize("fmt", FMTS)
@@ -32,8 +32,8 @@ def test_unaligned_scales_and_padded_rows(fmt):
 
 
 # (n, m) at 1280 or 672 values of K: together they take every plan of gemm_tile_plan on a 256-CU device
-PLANS = [(64, 70), (100, 49), (1100, 49), (1700, 66), (4310, 49), (5500, 60), (5600, 66), (8400, 66), (9940, 300),
-         (6360, 1000), (10960, 300)]
+PLANS = [(64, 5), (4331, 5), (8400, 9), (1420, 33), (4331, 20), (8400, 20), (2340, 200), (5340, 49), (8400, 33), (670, 768),
+         (8400, 66), (8400, 130), (11000, 130), (12330, 200), (11000, 260), (11000, 515)]
 
 
 @pytest.mark.parametrize("fmt", FMTS)
