@@ -116,9 +116,20 @@ def check(status, what):
     raise KompError(msg)
 
 
+_entries = {}
+
+
+def entry(name):
+    """An ABI function of the loaded library (looked up once)."""
+    fn = _entries.get(name)
+    if fn is None:
+        fn = _entries[name] = getattr(lib(), name)
+    return fn
+
+
 def call(name, *args):
     """Call an ABI function and raise on a nonzero status."""
-    check(getattr(lib(), name)(*args), name)
+    check(entry(name)(*args), name)
 
 
 def auto_plan(fmt_id, m, n, k, fused=False, mode=2):

@@ -46,6 +46,7 @@ for _f in FORMATS.values():
 MODES = {"bytes": 0, "dp4a": 2}  # mode 1 = dp4a emulated with shifts and multiplies
 FMT_ID = {"q4_0": 0, "tq2_0": 1, "q8_0": 2, "iq4_nl": 3, "q4_k": 4}
 _XB_F32 = ("q4_0", "tq2_0", "q4_k")  # formats whose gemv_f32 entry takes the XB (bsums) output
+_XB_NONE = {f: (None,) if f in _XB_F32 else () for f in FMT_ID}  # that argument, absent
 GEMM_MIN_M = {f: 4 for f in FMT_ID}  # columns from which gemv(..., block_n=None, mode=2) runs the matrix-core GEMM
 
 
@@ -108,9 +109,7 @@ def split_into(fmt, W, wq, ws, n, k):
     for t, name in ((wq, "wq"), (ws, "ws")):
         if t.device != W.device:
             raise _abi.KompArgumentError(f"{name} is on {t.device}, W on {W.device}")
-    fn = f"komp_{fmt}_split"
-    with torch.cuda.device(W.device):
-        _abi.call(fn, W.data_ptr(), wq.data_ptr(), ws.data_ptr(), n, k, wq.stride(0) if n else 16, _stream(W))
+    _launch(f"komp_{fmt}_split", W, W.data_ptr(), wq.data_ptr(), ws.data_ptr(), n, k, wq.stride(0) if n else 16)
 
 
 def split_q4_0(W, n, k):
@@ -164,12 +163,41 @@ def device():
     return "cuda" if torch.cuda.is_available() else "cpu"
 
 
-def _stream(t):
-    return ctypes_stream(t.device)
-
-
 def ctypes_stream(dev):
     return torch.cuda.current_stream(dev).cuda_stream
+
+
+# An eager call is mostly host time (15 us a call against 3 us of kernel at the decode shapes): its checks are one chain
+# of cheap attribute reads that must imply the full check, which runs, and names the fault, when any of them fails; the
+# current stream's handle comes without a Stream object (2.1 us), and the device is switched only if it is another one.
+_raw_stream = torch._C._cuda_getCurrentRawStream
+_current_device = torch._C._cuda_getDevice
+_Tensor, _U8, _I16, _I8, _F32 = torch.Tensor, torch.uint8, torch.int16, torch.int8, torch.float32
+
+
+def _launch(name, t, *args):
+    """Call a launching ABI entry on t's device, with that device's current stream as its last argument."""
+    dev = t.get_device()
+    if dev == _current_device():
+        st = _abi.entry(name)(*args, _raw_stream(dev))
+    else:
+        with torch.cuda.device(dev):
+            st = _abi.entry(name)(*args, _raw_stream(dev))
+    if st:
+        _abi.check(st, name)
+
+
+def _plane(t, dtype, shape, dev):
+    """True for a contiguous tensor of this dtype and shape on device number dev."""
+    return (isinstance(t, _Tensor) and t.is_cuda and t.dtype is dtype and t.shape == shape and t.is_contiguous()
+            and t.get_device() == dev)  # fmt: skip
+
+
+def _weights_fit(f, wq, ws, n, nblk, dev):
+    """True for split planes that pass every check of _check_weights, on device number dev."""
+    return (isinstance(wq, _Tensor) and wq.is_cuda and wq.dtype is _U8 and wq.dim() == 2 and wq.shape[0] == n
+            and wq.shape[1] >= nblk * f["qbytes"] and wq.stride(1) == 1 and wq.get_device() == dev
+            and _plane(ws, _I16, (n, nblk * f["sbytes"] // 2), dev))  # fmt: skip
 
 
 def _need(t, name, dtype, ndim=None):
@@ -188,30 +216,33 @@ def quantize(fmt, x, bb=4, bsums=False):
 
     src/komp/host.py:63-73.  With bsums=True (q8_K only) also returns XB int16 [M][K/16]."""
     act = FORMATS[fmt]["act"]
-    _need(x, "x", torch.float32, 2)
+    if not (isinstance(x, _Tensor) and x.is_cuda and x.dtype is _F32 and x.dim() == 2):
+        _need(x, "x", torch.float32, 2)
     x = x.contiguous()
     m, k = x.shape
     blk = 32 if act == "q8_0" else 256
     if k % blk:
         raise _abi.KompArgumentError(f"quantize {fmt}: K={k} is not a multiple of {blk}")
-    xq = torch.empty((m, k), dtype=torch.int8, device=x.device)
-    xd = torch.empty((m, k // blk), dtype=torch.float32, device=x.device)
-    s = _stream(x)
-    with torch.cuda.device(x.device):
-        if act == "q8_0":
-            if bsums:
-                raise _abi.KompArgumentError("bsums are a q8_K field; q8_0 has none")
-            _abi.call("komp_quant_q8_0", x.data_ptr(), xq.data_ptr(), xd.data_ptr(), m, k, bb, s)
-            return xq, xd
-        xb = torch.empty((m, k // 16), dtype=torch.int16, device=x.device) if bsums else None
-        _abi.call("komp_quant_q8_K", x.data_ptr(), xq.data_ptr(), xd.data_ptr(), xb.data_ptr() if bsums else None, m,
-                  k, s)  # fmt: skip
+    xq = x.new_empty((m, k), dtype=_I8)
+    xd = x.new_empty((m, k // blk))
+    if act == "q8_0":
+        if bsums:
+            raise _abi.KompArgumentError("bsums are a q8_K field; q8_0 has none")
+        _launch("komp_quant_q8_0", x, x.data_ptr(), xq.data_ptr(), xd.data_ptr(), m, k, bb)
+        return xq, xd
+    xb = x.new_empty((m, k // 16), dtype=_I16) if bsums else None
+    _launch("komp_quant_q8_K", x, x.data_ptr(), xq.data_ptr(), xd.data_ptr(), xb.data_ptr() if bsums else None, m, k)
     return (xq, xd, xb) if bsums else (xq, xd)
 
 
 def _check_gemv(fmt, wq, ws, xq, xd, n, k):
     """Validate the planes a GEMV reads (the C ABI sees raw pointers and cannot check buffer sizes)."""
     f = FORMATS[fmt]
+    nblk = k // f["block"]
+    if isinstance(xq, _Tensor) and xq.is_cuda and xq.dtype is _I8 and xq.dim() == 2 and xq.is_contiguous():
+        m, dev = xq.shape[0], xq.get_device()
+        if xq.shape[1] == k and _plane(xd, _F32, (m, nblk), dev) and _weights_fit(f, wq, ws, n, nblk, dev):
+            return m, nblk
     _need(wq, "wq", torch.uint8, 2)
     _need(ws, "ws", torch.int16, 2)
     _need(xq, "xq", torch.int8, 2)
@@ -237,11 +268,8 @@ def _check_gemv(fmt, wq, ws, xq, xd, n, k):
 def _launch_gemv(fmt, wq, ws, xq, xd, y, s, n, k, block_n, nb, mode, num_warps):
     if block_n is None:
         block_n, nb, num_warps = 0, 0, 0
-    fn = f"komp_{fmt}_gemv"
-    with torch.cuda.device(xq.device):
-        _abi.call(fn, wq.data_ptr(), ws.data_ptr(), xq.data_ptr(), xd.data_ptr(), y.data_ptr(),
-                  None if s is None else s.data_ptr(), xq.shape[0], n, k, wq.stride(0), block_n, nb, mode, num_warps,
-                  _stream(xq))  # fmt: skip
+    _launch(f"komp_{fmt}_gemv", xq, wq.data_ptr(), ws.data_ptr(), xq.data_ptr(), xd.data_ptr(), y.data_ptr(),
+            None if s is None else s.data_ptr(), xq.shape[0], n, k, wq.stride(0), block_n, nb, mode, num_warps)  # fmt: skip
 
 
 def gemv(fmt, wq, ws, xq, xd, n, k, block_n=32, nb=4, mode=0, num_warps=4, store_s=False):
@@ -249,17 +277,15 @@ def gemv(fmt, wq, ws, xq, xd, n, k, block_n=32, nb=4, mode=0, num_warps=4, store
 
     src/komp/host.py:76-85.  block_n=None lets the library choose block_n, nb and num_warps for the shape."""
     m, nblk = _check_gemv(fmt, wq, ws, xq, xd, n, k)
-    y = torch.empty((m, n), dtype=torch.float32, device=xq.device)
+    y = xd.new_empty((m, n))
     s = torch.zeros(_s_shape(fmt, m, n, nblk), dtype=torch.int32, device=xq.device) if store_s else None
     _launch_gemv(fmt, wq, ws, xq, xd, y, s, n, k, block_n, nb, mode, num_warps)
     return y, s
 
 
 def _launch_gemm(fmt, wq, ws, xq, xd, y, s, n, k):
-    fn = f"komp_{fmt}_gemm"
-    with torch.cuda.device(xq.device):
-        _abi.call(fn, wq.data_ptr(), ws.data_ptr(), xq.data_ptr(), xd.data_ptr(), y.data_ptr(),
-                  None if s is None else s.data_ptr(), xq.shape[0], n, k, wq.stride(0), _stream(xq))  # fmt: skip
+    _launch(f"komp_{fmt}_gemm", xq, wq.data_ptr(), ws.data_ptr(), xq.data_ptr(), xd.data_ptr(), y.data_ptr(),
+            None if s is None else s.data_ptr(), xq.shape[0], n, k, wq.stride(0))  # fmt: skip
 
 
 def gemm(fmt, wq, ws, xq, xd, n, k, store_s=False):
@@ -269,7 +295,7 @@ def gemm(fmt, wq, ws, xq, xd, n, k, store_s=False):
     weights are read once per 64 columns.  gemv(..., block_n=None, mode=2) runs this kernel from GEMM_MIN_M columns
     on."""
     m, nblk = _check_gemv(fmt, wq, ws, xq, xd, n, k)
-    y = torch.empty((m, n), dtype=torch.float32, device=xq.device)
+    y = xd.new_empty((m, n))
     s = torch.zeros(_s_shape(fmt, m, n, nblk), dtype=torch.int32, device=xq.device) if store_s else None
     _launch_gemm(fmt, wq, ws, xq, xd, y, s, n, k)
     return y, s
@@ -332,16 +358,15 @@ def quantize_into(fmt, x, xq, xd, xb=None, bb=4):
     blk = 32 if act == "q8_0" else 256
     if tuple(xq.shape) != (m, k) or tuple(xd.shape) != (m, k // blk):
         raise _abi.KompArgumentError(f"quantize_into: xq must be [{m}][{k}] and xd [{m}][{k // blk}]")
-    with torch.cuda.device(x.device):
-        if act == "q8_0":
-            _abi.call("komp_quant_q8_0", x.data_ptr(), xq.data_ptr(), xd.data_ptr(), m, k, bb, _stream(x))
-        else:
-            if xb is not None:
-                _need(xb, "xb", torch.int16, 2)
-                if tuple(xb.shape) != (m, k // 16) or not xb.is_contiguous():
-                    raise _abi.KompArgumentError(f"quantize_into: xb must be a contiguous [{m}][{k // 16}] plane")
-            _abi.call("komp_quant_q8_K", x.data_ptr(), xq.data_ptr(), xd.data_ptr(),
-                      None if xb is None else xb.data_ptr(), m, k, _stream(x))  # fmt: skip
+    if act == "q8_0":
+        _launch("komp_quant_q8_0", x, x.data_ptr(), xq.data_ptr(), xd.data_ptr(), m, k, bb)
+    else:
+        if xb is not None:
+            _need(xb, "xb", torch.int16, 2)
+            if tuple(xb.shape) != (m, k // 16) or not xb.is_contiguous():
+                raise _abi.KompArgumentError(f"quantize_into: xb must be a contiguous [{m}][{k // 16}] plane")
+        _launch("komp_quant_q8_K", x, x.data_ptr(), xq.data_ptr(), xd.data_ptr(), None if xb is None else xb.data_ptr(),
+                m, k)  # fmt: skip
 
 
 def gemv_into(fmt, wq, ws, xq, xd, y, n, k, block_n=None, nb=4, mode=2, num_warps=4, s=None):
@@ -374,11 +399,8 @@ def _check_weights(fmt, wq, ws, n, k):
     return nblk
 
 
-def gemv_f32_into(fmt, wq, ws, x, y, n, k, block_n=None, nb=4, mode=2, num_warps=4, s=None, xq=None, xd=None,
-                  xb=None):  # fmt: skip
-    """Quantize-and-GEMV in one launch into preallocated outputs: x f32 [M][K] -> y f32 [M][N] (and s, and the q8
-    planes xq / xd / xb when given, as quantize() would return them).  Bit-identical to quantize() then gemv() with
-    the same knobs."""
+def _check_gemv_f32(fmt, wq, ws, x, y, n, k, s, xq, xd, xb):
+    """Validate the tensors of a gemv_f32_into call."""
     nblk = _check_weights(fmt, wq, ws, n, k)
     _need(x, "x", torch.float32, 2)
     if x.shape[1] != k or not x.is_contiguous():
@@ -402,16 +424,28 @@ def gemv_f32_into(fmt, wq, ws, x, y, n, k, block_n=None, nb=4, mode=2, num_warps
     for t, name in ((wq, "wq"), (ws, "ws"), (y, "y")):
         if t.device != x.device:
             raise _abi.KompArgumentError(f"{name} is on {t.device}, x on {x.device}")
+
+
+def gemv_f32_into(fmt, wq, ws, x, y, n, k, block_n=None, nb=4, mode=2, num_warps=4, s=None, xq=None, xd=None,
+                  xb=None):  # fmt: skip
+    """Quantize-and-GEMV in one launch into preallocated outputs: x f32 [M][K] -> y f32 [M][N] (and s, and the q8
+    planes xq / xd / xb when given, as quantize() would return them).  Bit-identical to quantize() then gemv() with
+    the same knobs."""
+    f = FORMATS[fmt]
+    if not (s is None and xq is None and xd is None and xb is None and isinstance(x, _Tensor) and x.is_cuda
+            and x.dtype is _F32 and x.dim() == 2 and x.shape[1] == k and x.is_contiguous()
+            and _plane(y, _F32, (x.shape[0], n), x.get_device())
+            and _weights_fit(f, wq, ws, n, k // f["block"], x.get_device())):  # fmt: skip
+        _check_gemv_f32(fmt, wq, ws, x, y, n, k, s, xq, xd, xb)
+    m = x.shape[0]
     if block_n is None:
         block_n, nb, num_warps = 0, 0, 0
-    fn = f"komp_{fmt}_gemv_f32"
-    ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    planes = (ptr(xq), ptr(xd), ptr(xb)) if fmt in _XB_F32 else (ptr(xq), ptr(xd))  # the others: no XB
+    planes = (xq, xd, xb) if fmt in _XB_F32 else (xq, xd)  # the others: no XB
     if xb is not None and FORMATS[fmt]["act"] != "q8_K":
         raise _abi.KompArgumentError("xb (bsums) is a q8_K plane; pass None for q8_0 activations")
-    with torch.cuda.device(x.device):
-        _abi.call(fn, wq.data_ptr(), ws.data_ptr(), x.data_ptr(), y.data_ptr(), ptr(s), *planes, m, n, k, wq.stride(0),
-                  block_n, nb, mode, num_warps, _stream(x))  # fmt: skip
+    _launch(f"komp_{fmt}_gemv_f32", x, wq.data_ptr(), ws.data_ptr(), x.data_ptr(), y.data_ptr(),
+            *(None if t is None else t.data_ptr() for t in (s, *planes)), m, n, k, wq.stride(0), block_n, nb, mode,
+            num_warps)  # fmt: skip
 
 
 def gemv_f32(fmt, wq, ws, x, n, k, block_n=None, nb=4, mode=2, num_warps=4, store_s=False, return_q=False):
@@ -421,13 +455,20 @@ def gemv_f32(fmt, wq, ws, x, n, k, block_n=None, nb=4, mode=2, num_warps=4, stor
     equals quantize() followed by gemv() with the same knobs bit for bit, with one dispatch instead of two
     (block_n=None plans this launch with auto_config(..., fused=True)).  return_q also returns the q8
     planes (and the q8_K bsums).  No reference counterpart (the reference launches the two kernels separately)."""
-    _need(x, "x", torch.float32, 2)
+    if not (isinstance(x, _Tensor) and x.is_cuda and x.dtype is _F32 and x.dim() == 2):
+        _need(x, "x", torch.float32, 2)
     x = x.contiguous()
     m = x.shape[0]
     blk = FORMATS[fmt]["block"]
     if k % blk:
         raise _abi.KompArgumentError(f"{fmt}: K={k} is not a multiple of {blk}")
-    y = torch.empty((m, n), dtype=torch.float32, device=x.device)
+    y = x.new_empty((m, n))
+    if not (store_s or return_q) and x.shape[1] == k and _weights_fit(FORMATS[fmt], wq, ws, n, k // blk, x.get_device()):
+        if block_n is None:
+            block_n, nb, num_warps = 0, 0, 0
+        _launch(f"komp_{fmt}_gemv_f32", x, wq.data_ptr(), ws.data_ptr(), x.data_ptr(), y.data_ptr(), None, None, None,
+                *_XB_NONE[fmt], m, n, k, wq.stride(0), block_n, nb, mode, num_warps)  # fmt: skip
+        return y, None
     s = torch.zeros(_s_shape(fmt, m, n, k // blk), dtype=torch.int32, device=x.device) if store_s else None
     q = None
     if return_q:
@@ -480,11 +521,9 @@ def gemv_multi_into(fmt, mats, ys, k, xq=None, xd=None, x=None, block_n=None, nb
     yps = P(*(y.data_ptr() for y in ys))
     ns = I64(*(n for _, _, n in mats))
     sws = I64(*(w.stride(0) for w, _, _ in mats))
-    fn = f"komp_{fmt}_gemv_multi"
     ptr = lambda t: None if t is None else t.data_ptr()  # noqa: E731
-    with torch.cuda.device(ref.device):
-        _abi.call(fn, cnt, wqs, wss, yps, ns, sws, ptr(xq), ptr(xd), ptr(x), m, k, block_n, nb, mode, num_warps,
-                  _stream(ref))  # fmt: skip
+    _launch(f"komp_{fmt}_gemv_multi", ref, cnt, wqs, wss, yps, ns, sws, ptr(xq), ptr(xd), ptr(x), m, k, block_n, nb, mode,
+            num_warps)  # fmt: skip
 
 
 def gemv_multi(fmt, mats, k, xq=None, xd=None, x=None, block_n=None, nb=4, mode=2, num_warps=4):
@@ -531,9 +570,7 @@ def dp4a_probe(a, b, c, mode=2):
         _need(t, name, torch.int32, 1)
     a, b, c = a.contiguous(), b.contiguous(), c.contiguous()
     out = torch.empty_like(a)
-    with torch.cuda.device(a.device):
-        _abi.call("komp_dp4a_probe", a.data_ptr(), b.data_ptr(), c.data_ptr(), out.data_ptr(), a.numel(), mode,
-                  _stream(a))  # fmt: skip
+    _launch("komp_dp4a_probe", a, a.data_ptr(), b.data_ptr(), c.data_ptr(), out.data_ptr(), a.numel(), mode)
     return out
 
 
@@ -551,8 +588,7 @@ def stream_read_into(src, nbytes, out):
     _need(out, "out", torch.int32, 1)
     if out.numel() < stream_read_words(nbytes):
         raise _abi.KompArgumentError(f"out needs {stream_read_words(nbytes)} words")
-    with torch.cuda.device(src.device):
-        _abi.call("komp_stream_read", src.data_ptr(), nbytes, out.data_ptr(), _stream(src))
+    _launch("komp_stream_read", src, src.data_ptr(), nbytes, out.data_ptr())
 
 
 def stream_read(src):
@@ -569,8 +605,7 @@ def q4_0_decode(wq):
     wq = wq.contiguous()
     r = wq.shape[0]
     out = torch.empty((r, 32), dtype=torch.int32, device=wq.device)
-    with torch.cuda.device(wq.device):
-        _abi.call("komp_q4_0_decode", wq.data_ptr(), out.data_ptr(), r, _stream(wq))
+    _launch("komp_q4_0_decode", wq, wq.data_ptr(), out.data_ptr(), r)
     return out
 
 
@@ -580,6 +615,5 @@ def tq2_0_decode(wq):
     wq = wq.contiguous()
     nblk = wq.shape[0]
     out = torch.empty((nblk, 256), dtype=torch.int32, device=wq.device)
-    with torch.cuda.device(wq.device):
-        _abi.call("komp_tq2_0_decode", wq.data_ptr(), out.data_ptr(), nblk, _stream(wq))
+    _launch("komp_tq2_0_decode", wq, wq.data_ptr(), out.data_ptr(), nblk)
     return out
