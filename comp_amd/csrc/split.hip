@@ -7,13 +7,17 @@
 // order) and WS i16 [N][K/blk] (the f16 bit patterns; Q4_K: [N][8 K/256], each block's first 16 bytes).  Pure byte
 // movement, so the planes equal host.split's bit for bit.
 //
-// One thread per 16-byte chunk of WQ (Q4_0, IQ4_NL: one per block, Q8_0: two, TQ2_0: four, Q4_K: eight).  A chunk's 16 source
-// bytes start at an address that is 2 mod 4 for every other block (18-, 34- and 66-byte blocks), so the thread loads the aligned words that
-// cover them and funnel-shifts them into place (v_alignbyte_b32); consecutive threads read consecutive 16-18 byte
-// windows, so each wave's loads cover contiguous memory.  The loads go through a buffer descriptor whose range ends at
-// the launch's last byte, so nothing is read past the tensor.
-// The thread of chunk 0 also moves the block's scale-plane bytes (2, or Q4_K's 16 in one 16-byte load and store).  HBM-bound: it reads each ggml byte once and writes
-// each plane byte once.
+// A workgroup moves 256 16-byte chunks of WQ, one a thread (Q4_0, IQ4_NL: a block each, Q8_0: half a block, TQ2_0: a
+// quarter, Q4_K: an eighth).  Their ggml bytes (16.5 to 18 a chunk) are a whole number of 16-byte pieces at a 16-byte
+// offset: they are read in such pieces and go through LDS, where a chunk's bytes start 0 or 2 bytes into a dword (block
+// sizes and offsets are even): five dwords funnel-shifted into place (v_alignbyte_b32).  The thread of a block's chunk 0
+// also moves its scale-plane bytes (2, or Q4_K's 16 in one store).
+//
+// HBM-bound: it reads each ggml byte once and writes each plane byte once.  No cache line is needed twice and the planes
+// of a whole model are past every cache by the first token, so loads and stores are non-temporal.  Q4_0, buffers that
+// rotate past the caches, us at 128256 x 4096 (591 MB in and out) / 14336 x 4096 / 4096 x 4096: a thread reading its own 18
+// bytes in dwords 105.5 / 14.8 / 5.0; through LDS 97.9 / 13.3 / 4.6; non-temporal as well 89.6 (6.6 TB/s; a plain copy of
+// 16 bytes a lane 5.6) / 12.0 / 4.4; four tiles a workgroup 94.2 / 12.1 / 4.3.
 #include <hip/hip_ext.h>
 
 #include "komp_device.h"
@@ -24,6 +28,8 @@ namespace split_impl {
 
 constexpr int kRsrcWord3 = 0x00020000;  // buffer descriptor word 3 on gfx9: 32-bit data, no swizzle
 constexpr int kThreads = 256;
+constexpr int kNt = 2;                  // buffer load cache policy: non-temporal
+constexpr unsigned kOob = 0x7FFFFFF0u;  // an offset past every descriptor's range: the load returns zeros
 
 // chunks: WQ chunks in this launch (blocks * chunks per block); nblk: blocks per row; cpb_log2: log2(chunks per
 // block); nbytes, qoff, soff: the ggml block's size, quant offset and scale offset; wbytes: the launch's ggml bytes.
@@ -31,33 +37,50 @@ constexpr int kThreads = 256;
 __global__ void __launch_bounds__(kThreads)
 split_kernel(int chunks, int nblk, int cpb_log2, int nbytes, int qoff, int soff, int sbytes, int wbytes, int64_t SW,
              const uint8_t* __restrict__ W, uint8_t* __restrict__ WQ, int16_t* __restrict__ WS) {
-  const int t = blockIdx.x * kThreads + threadIdx.x;
-  if (t >= chunks) return;
+  constexpr int kPieces = 2;  // 16-byte pieces a thread: the workgroup's at most 18 bytes a chunk are at most 288
+  __shared__ __align__(16) unsigned char lds[kPieces * kThreads * 16];
   const auto w = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(W), 0, wbytes, kRsrcWord3);
-  const int b = t >> cpb_log2;            // block within the launch
-  const int c = t & ((1 << cpb_log2) - 1);  // chunk within the block
+  const int tid = threadIdx.x;
+  const int blocks = kThreads >> cpb_log2;  // of the workgroup
+  const int b0 = blockIdx.x * blocks;
+  const unsigned first = static_cast<unsigned>(b0) * nbytes;
+  const int bytes = min(blocks * nbytes, wbytes - static_cast<int>(first));
+  u32x4 v[kPieces];
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) {
+    const int o = 16 * (i * kThreads + tid);
+    v[i] = __builtin_amdgcn_raw_buffer_load_b128(w, o + 16 <= bytes ? first + o : kOob, 0, kNt);
+  }
+#pragma unroll
+  for (int i = 0; i < kPieces; ++i) *reinterpret_cast<u32x4*>(lds + 16 * (i * kThreads + tid)) = v[i];
+  __syncthreads();
+  const int tail = bytes & 15;  // the launch's last bytes, short of a piece: 2 bytes a thread
+  if (tail != 0) {              // the same for the whole workgroup
+    if (2 * tid < tail)
+      *reinterpret_cast<uint16_t*>(lds + bytes - tail + 2 * tid) =
+          __builtin_amdgcn_raw_buffer_load_b16(w, first + bytes - tail + 2 * tid, 0, 0);
+    __syncthreads();
+  }
+  if (blockIdx.x * kThreads + tid >= static_cast<unsigned>(chunks)) return;
+  const int lb = tid >> cpb_log2;             // block within the workgroup
+  const int c = tid & ((1 << cpb_log2) - 1);  // chunk within the block
+  const int b = b0 + lb;
   const int row = b / nblk;
   const int col = b - row * nblk;
-  // src is even (block sizes and offsets are even), so the window starts 0 or 2 bytes into its first dword and needs
-  // at most the low half of a fifth one.  That half is a 2-byte load: a 4-byte load that crosses the descriptor's end
-  // returns zero whole, which would drop the last block's last two bytes.
-  const unsigned src = static_cast<unsigned>(b * nbytes + qoff + 16 * c);
-  const unsigned a = src & ~3u;
-  const unsigned sh = src & 3u;
-  unsigned d[5];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) d[i] = __builtin_amdgcn_raw_buffer_load_b32(w, a + 4 * i, 0, 0);
-  d[4] = __builtin_amdgcn_raw_buffer_load_b16(w, a + 16, 0, 0);
+  const unsigned src = static_cast<unsigned>(lb * nbytes + qoff + 16 * c);
+  const unsigned* const d = reinterpret_cast<const unsigned*>(lds + (src & ~3u));
   u32x4 o;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = __builtin_amdgcn_alignbyte(d[i + 1], d[i], sh);
-  *reinterpret_cast<u32x4*>(WQ + row * SW + (static_cast<int64_t>(col) << (cpb_log2 + 4)) + 16 * c) = o;
+  for (int j = 0; j < 4; ++j) o[j] = __builtin_amdgcn_alignbyte(d[j + 1], d[j], src & 3u);
+  uint8_t* const wq = WQ + row * SW + (static_cast<int64_t>(col) << (cpb_log2 + 4)) + 16 * c;
+  __builtin_nontemporal_store(o, reinterpret_cast<u32x4*>(wq));
   if (c == 0) {
-    const unsigned so = static_cast<unsigned>(b * nbytes + soff);
+    const unsigned char* const so = lds + lb * nbytes + soff;
     if (sbytes == 16)  // Q4_K: 144-byte blocks, so the 16 bytes start 16-byte aligned
-      *reinterpret_cast<u32x4*>(WS + 8 * b) = __builtin_amdgcn_raw_buffer_load_b128(w, so, 0, 0);
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(so),
+                                  reinterpret_cast<u32x4*>(WS + 8 * static_cast<int64_t>(b)));
     else
-      WS[b] = static_cast<int16_t>(__builtin_amdgcn_raw_buffer_load_b16(w, so, 0, 0));
+      __builtin_nontemporal_store(*reinterpret_cast<const int16_t*>(so), WS + b);
   }
 }
 
@@ -76,6 +99,7 @@ hipError_t launch_split(int fmt, const uint8_t* w, uint8_t* wq, int16_t* ws, int
   const int64_t row_bytes = nblk * nbytes;
   int64_t rows_per = row_bytes > 0 ? (int64_t{1} << 30) / row_bytes : n;
   if (rows_per < 1) rows_per = 1;
+  if (rows_per >= 8) rows_per &= ~int64_t{7};  // each batch starts 16-byte aligned to the first
   for (int64_t r0 = 0; r0 < n; r0 += rows_per) {
     const int64_t rows = n - r0 < rows_per ? n - r0 : rows_per;
     const int64_t chunks = rows * nblk << cpb_log2;

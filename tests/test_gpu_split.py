@@ -38,6 +38,23 @@ def test_split_matches_oracle(fmt, shape):
 
 
 @pytest.mark.parametrize("fmt", ["q4_0", "tq2_0", "q8_0", "iq4_nl", "q4_k"])
+@pytest.mark.parametrize("rows,chunks", [(1, 256), (1, 264), (3, 248), (1, 8), (4, 128), (4099, 136)])
+def test_split_tile_edges(fmt, rows, chunks):
+    """Rows of `chunks` 16-byte chunks: one workgroup's 256 and its neighbours, launches that end with a whole workgroup
+    or inside one, short of a 16-byte piece."""
+    blk, nbytes, qbytes = NBYTES[fmt]
+    nb = chunks * 16 // qbytes
+    rng = np.random.default_rng(chunks)
+    W = rng.integers(0, 256, rows * nb * nbytes, dtype=np.uint8)
+    rq, rs = O.split(fmt, W.tobytes(), rows, nb * blk)
+    print(f"split {fmt} n={rows} k={nb * blk}", flush=True)
+    base = torch.zeros(W.size + 12, dtype=torch.uint8, device="cuda")
+    base[4 : 4 + W.size] = dev(W)
+    wq, ws = host.split_device(fmt, base[4 : 4 + W.size], rows, nb * blk)
+    assert np.array_equal(wq.cpu().numpy(), rq) and np.array_equal(ws.cpu().numpy(), rs)
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "tq2_0", "q8_0", "iq4_nl", "q4_k"])
 def test_split_padded_rows_and_offset_input(fmt):
     n, nb = 29, 11
     blk, nbytes, qbytes = NBYTES[fmt]
