@@ -402,19 +402,20 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 // The tiled GEMM (gemm_tile.h) takes every batch whose rows are long enough.  Measured on MI355X against gemm.hip's kernel
 // (graph replays, cold weights) over 10 shapes (127 x 4096 to 28672 x 4096) and 14 column counts from 4 to 2048 it is
 // faster at nearly all of them: Q4_0 28672 x 4096 at 16 columns 30.8 -> 20.1 us, 14336 x 4096 at 64 columns 35 -> 24, at
-// 512 columns 385 -> 116, Q8_0 14336 x 4096 at 16 columns 24.3 -> 14.1, TQ2_0 6912 x 2560 at 8 columns 6.3 -> 4.7, at 2048
+// 512 columns 385 -> 105, Q8_0 14336 x 4096 at 16 columns 24.3 -> 14.1, TQ2_0 6912 x 2560 at 8 columns 6.3 -> 4.7, at 2048
 // columns 326 -> 61, Q4_K 4096 x 14336 at 1001 columns 561 -> 181.  gemm.hip's kernel keeps
 //   rows of at most 4 K steps, which are over before the tile's staging pays;
 //   Q4_K's few columns, whose scale products the tile multiplies into the weights once per column group: up to 8 columns
-//     (4096 x 14336 12.8 us against 15.3, 28672 x 4096 at 4 columns 22.9 against 24.8), up to 16 over at most 2 row tiles
-//     a CU (2560 x 6912 at 16 columns 8.8 against 9.4); up to 32 where two column groups are just past a workgroup a CU
-//     (2560 x 6912 at 24 columns 11.3 against 13.7); and 49-64 columns over at most 3 row tiles a CU (4096 x 14336 40 us
-//     in one group of 64 columns and in the tile's narrower ones).
+//     (4096 x 14336 13.3 us against 16.3, 28672 x 4096 at 5 columns 24.8 against 25.3); up to 16 over at most 2 row tiles a
+//     CU where rows are long or few (2560 x 6912 at 16 columns 9.2 against 9.8, 127 x 2816 5.1 against 6.1; 4096 x 4096 7.6
+//     against 7.0 goes to the tile); up to 32 where two column groups are just past a workgroup a CU (2560 x 6912 at 24
+//     columns 11.6 against 12.8).
 //
 // The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
-// launch has 3 us besides.  The constants are a least-squares fit over those shapes; the plan they pick is within 1% of
-// the fastest one in the geometric mean.
+// launch has 3 us besides.  The constants are fitted to 12 column counts from 5 to 2048 over 8 or 9 shapes a format (127 to
+// 28672 rows); the plan they pick is within 1-2.5% of the fastest of all 22 measured ones in the geometric mean, and a format
+// leaves out the plans that this does not need.
 struct TileCost {
   TilePlan p;
   struct {
@@ -423,18 +424,23 @@ struct TileCost {
   } f[4];  // Q4_0 and IQ4_NL, TQ2_0, Q8_0, Q4_K
 };
 constexpr TileCost kTileCosts[] = {
-    {{1, 1, 1, 8}, {{2, 0.f, 0.58f}, {2, 0.f, 0.74f}, {2, 0.f, 0.65f}, {1, 0.f, 0.99f}}},
-    {{1, 2, 1, 8}, {{2, 0.f, 0.87f}, {1, 0.f, 1.22f}, {2, 0.f, 1.06f}, {1, 0.f, 1.37f}}},
-    {{1, 2, 1, 4}, {{4, 0.11f, 0.41f}, {3, 0.08f, 0.45f}, {4, 0.04f, 0.53f}, {3, 0.30f, 0.47f}}},
-    {{2, 1, 2, 4}, {{2, 0.13f, 0.80f}, {2, 0.f, 0.78f}, {1, 0.f, 0.99f}, {1, 0.f, 1.04f}}},
-    {{2, 2, 2, 4}, {{1, 0.f, 1.60f}, {1, 0.f, 1.41f}, {1, 0.f, 1.83f}, {1, 0.f, 1.59f}}},
-    {{2, 1, 4, 4}, {{1, 0.f, 1.82f}, {1, 0.f, 1.62f}, {1, 0.f, 1.88f}, {1, 0.f, 1.61f}}},
-    {{4, 1, 4, 2}, {{2, 0.07f, 1.11f}, {2, 0.f, 0.97f}, {1, 0.f, 1.28f}, {1, 0.f, 1.19f}}},
-    {{4, 1, 8, 2}, {{1, 0.f, 2.39f}, {1, 0.f, 1.84f}, {1, 0.f, 2.42f}, {1, 0.f, 1.92f}}},
-    {{4, 2, 4, 1}, {{3, 0.58f, 0.73f}, {2, 0.36f, 0.62f}, {3, 0.54f, 0.85f}, {2, 0.52f, 0.65f}}},
-    {{4, 2, 8, 1}, {{2, 1.14f, 1.22f}, {2, 0.61f, 1.08f}, {1, 0.f, 2.29f}, {0, 0.f, 0.f}}},
-    {{4, 2, 8, 2}, {{1, 0.f, 3.59f}, {1, 0.f, 2.84f}, {1, 0.f, 3.77f}, {0, 0.f, 0.f}}},
-    {{8, 1, 8, 1}, {{1, 0.f, 1.92f}, {1, 0.f, 1.44f}, {1, 0.f, 2.03f}, {1, 0.f, 1.63f}}},
+    {{1, 1, 1, 8}, {{2, 0.f, 0.60f}, {1, 0.f, 0.78f}, {1, 0.f, 0.80f}, {1, 0.f, 0.88f}}},
+    {{1, 2, 1, 8}, {{2, 0.f, 0.82f}, {1, 0.f, 1.11f}, {3, 0.f, 1.08f}, {1, 0.f, 1.40f}}},
+    {{1, 2, 1, 4}, {{4, 0.11f, 0.39f}, {2, 0.20f, 0.39f}, {2, 0.10f, 0.47f}, {3, 0.33f, 0.50f}}},
+    {{1, 1, 1, 4}, {{2, 0.16f, 0.18f}, {2, 0.24f, 0.21f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
+    {{2, 1, 1, 4}, {{0, 0.f, 0.f}, {2, 0.11f, 0.45f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
+    {{2, 2, 1, 4}, {{2, 0.21f, 0.69f}, {2, 0.03f, 0.95f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
+    {{2, 1, 2, 4}, {{2, 0.12f, 0.73f}, {2, 0.06f, 0.77f}, {0, 0.f, 0.f}, {1, 0.f, 0.91f}}},
+    {{2, 2, 2, 4}, {{1, 0.f, 1.38f}, {1, 0.f, 1.41f}, {1, 0.f, 1.73f}, {1, 0.f, 1.70f}}},
+    {{2, 1, 4, 4}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {1, 0.f, 1.56f}}},
+    {{4, 1, 4, 2}, {{2, 0.07f, 0.99f}, {1, 0.f, 0.99f}, {4, 0.22f, 1.05f}, {1, 0.f, 1.10f}}},
+    {{4, 2, 4, 2}, {{1, 0.f, 1.83f}, {1, 0.f, 1.71f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
+    {{4, 2, 4, 1}, {{3, 0.54f, 0.68f}, {0, 0.f, 0.f}, {4, 0.45f, 0.76f}, {0, 0.f, 0.f}}},
+    {{4, 1, 8, 2}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {1, 0.f, 1.65f}}},
+    {{4, 2, 8, 1}, {{2, 1.10f, 1.17f}, {4, 0.35f, 1.10f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
+    {{4, 2, 8, 2}, {{1, 0.f, 3.54f}, {0, 0.f, 0.f}, {2, 0.05f, 3.51f}, {0, 0.f, 0.f}}},
+    {{8, 1, 8, 1}, {{0, 0.f, 0.f}, {1, 0.f, 1.35f}, {3, 0.43f, 1.57f}, {1, 0.f, 1.39f}}},
+    {{8, 2, 8, 1}, {{1, 0.f, 3.07f}, {1, 0.f, 2.24f}, {1, 0.f, 3.43f}, {0, 0.f, 0.f}}},
 };
 
 // False when the call stays on gemm.hip's kernel: by the rules above, or past the tile's 32-bit buffer offsets (128 rows
@@ -445,8 +451,8 @@ bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePl
   const int64_t cus = device_cus();
   if (steps <= 4 || n < 1) return false;
   if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
-  if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus) || (m <= 32 && n > 8 * cus && n <= 12 * cus) ||
-                          (m > 48 && m <= 64 && n <= 48 * cus)))
+  if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus && (nblk > 24 || n <= cus)) ||
+                          (m <= 32 && n > 8 * cus && n <= 12 * cus)))
     return false;
   const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : fmt == FMT_Q4_K ? 3 : 0;
   double best = -1;

@@ -3,16 +3,19 @@
 // instruction takes, instead of read and rearranged by every wave.
 //
 // Bound.  Each block's exact integer dot is scaled in f32 by its own d_w * d_x, so the VALU runs a fixed number of
-// instructions per output and block beside the matrix cores.  The batched kernel in gemm.hip spends per 16x16 tile and
-// 32-value block 12 of them on the scaling (convert, multiply, fused multiply-add of 4 outputs a lane) and about as
+// instructions per output and block beside the matrix cores, and a matrix instruction of 16 cycles takes about two VALU
+// issues from them (measured: 8 of them 65 ns, 32 v_fma_f32 61, both 92).  The batched kernel in gemm.hip spends per
+// 16x16 tile and 32-value block 12 VALU instructions on the scaling (convert, multiply, fused multiply-add of 4 outputs a lane) and about as
 // many on rearranging operands, re-read per 64 columns.  Here:
 //   32-value blocks (Q4_0, IQ4_NL, Q8_0) and Q4_K go through v_mfma_f32_16x16x32_f16 with both operands as integers in
 //     f16.  Every product and partial sum is an integer below 2^24 (Q8_0: 32 * 128 * 128 = 2^19; Q4_K: the 6-bit
 //     sub-block scale times the nibble, at most 945, over half a block: 945 * 128 * 128 = 15.5 M; the two halves are
 //     added in f32, which rounds where the integer sum's conversion would), so the f32 result is the exact block dot,
-//     whatever order the matrix core adds in, and needs no conversion: 8 instructions instead of
-//     12.  One f16 instruction covers a 32-value block in the time the int8 one does (its int8 form of K 32 has no
-//     higher rate).
+//     whatever order the matrix core adds in, and needs no conversion: 8 instructions instead of 12.  The products
+//     d_w * d_x of four tiles are one v_mfma_f32_16x16x1_4b_f32 (16 multiplications take 30 ns of the VALU, it 15, and the
+//     scales reach it as a dword a lane instead of four and one), which leaves 4 instructions: Q4_0 14336 x 4096 at 512
+//     columns 117 -> 105 us (with 256-row tiles), Q4_K 4096 x 14336 at 1001 columns 192 -> 188 a call.  One f16
+//     instruction covers a 32-value block in the time the int8 one does (its int8 form of K 32 has no higher rate).
 //   TQ2_0's 256-value blocks stay on v_mfma_i32_16x16x64_i8 (twice the f16 rate; the scaling is 1/8 as often).
 //
 //   With one column tile (up to 16 columns) the 32-value blocks go through v_mfma_i32_16x16x32_i8: there the way of the
@@ -35,8 +38,8 @@
 // crossed with g put those on different banks.  (Padding every unit row by 16 bytes instead left the reads with 42% of
 // their LDS cycles in conflicts.)
 //
-// What it reaches: IQ4_NL 14336 x 4096 at 2048 columns issues VALU instructions 81% of the time (about 890 a wave and
-// step, 512 of them the scaling), matrix instructions 23%; TQ2_0 6912 x 2560 at 2048 columns 1.19 POP/s.
+// What it reaches: Q4_0 14336 x 4096 at 512 columns 105 us, of which the VALU's issue slots (matrix instructions
+// included) are about 95 at the 7/8 of its CUs that the tiles fill evenly; TQ2_0 6912 x 2560 at 2048 columns 64 us.
 #pragma once
 
 #include <hip/hip_ext.h>
@@ -53,6 +56,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kRsrcWord3 = 0x00020000;  // buffer descriptor word 3 on gfx9: 32-bit data, no swizzle
 constexpr unsigned kOob = 0x7FFFFFF0u;  // an offset past every descriptor's range: the load returns zeros
@@ -77,6 +81,12 @@ __device__ __forceinline__ f16x8 frag(unsigned a, unsigned b, unsigned c, unsign
   return __builtin_bit_cast(f16x8, u32x4{a, b, c, d});
 }
 
+// Four 16 x 16 outer products in C layout: block b (dwords 4b..4b+3) holds a of lanes 16b.. times b of lanes 16b..,
+// rounded to f32 once, as the multiplication would.
+__device__ __forceinline__ f32x16 outer4(float a, float b) {
+  return __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, f32x16{}, 0, 0, 0);
+}
+
 // LDS bytes of one K group's part: two activation buffers, two d_x buffers and (Q4_K) two buffers of 16-value sums; and
 // of one wave's scales.
 constexpr bool blk32(int fmt) { return fmt == FMT_Q4_0 || fmt == FMT_IQ4_NL || fmt == FMT_Q8_0; }
@@ -87,7 +97,8 @@ struct Lds {
   static constexpr int kRow = 16 * CN * kUnit;             // a unit row: a unit a column
   static constexpr int kPiece = 4 * kRow + 64;             // the four groups' rows of a piece, and the pad
   static constexpr int kBuf = 4 * kPiece;
-  static constexpr int kDx = 16 * CN * (FMT == FMT_TQ2_0 || FMT == FMT_Q4_K ? 1 : 4) * 4;
+  static constexpr int kDxRow = 16 * CN + 16;  // 32-value blocks: d_x lies [block][column], 16 banks apart block by block
+  static constexpr int kDx = FMT == FMT_TQ2_0 || FMT == FMT_Q4_K ? 16 * CN * 4 : 4 * kDxRow * 4;
   static constexpr int kSums = FMT == FMT_Q4_K ? 2 * kRow : 0;
   static constexpr int kGroup = 2 * (kBuf + kDx + kSums);
   // one wave's part: 64 weight bytes of each row, f32 scales (4 blocks of 16 rows a tile; TQ2_0 one; Q4_K d and dmin)
@@ -281,7 +292,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
 #pragma unroll
     for (int i = 0; i < DI; ++i) {
       const int idx = i * T + tid;
-      if (DI * T == DN || idx < DN) dxb[idx] = a.d[i];
+      if (DI * T == DN || idx < DN) dxb[BLK32 ? (idx & 3) * L::kDxRow + (idx >> 2) : idx] = a.d[i];
     }
   };
 
@@ -322,9 +333,11 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       long x[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const long*>(b + j * L::kPiece);
-      const f32x4 dx = *reinterpret_cast<const f32x4*>(dxp + r16 * 16);
       i32x4 corr[4], cc[2][WN];
-      f32x4 dw[2][WN];
+      f32x16 pr[WN];  // d_w * d_x: instruction block j is the step's block j
+      const float dx = reinterpret_cast<const float*>(dxp)[g * L::kDxRow + r16];
+#pragma unroll
+      for (int t = 0; t < WN; ++t) pr[t] = outer4(scl[t * 64 + lane], dx);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         corr[j] = i32x4{0, 0, 0, 0};
@@ -339,7 +352,7 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           for (int r = 0; r < 4; ++r) cf[r] = static_cast<float>(cc[j & 1][t][r]);
           if (STORE_S && 4 * s + j < nblk && s < s1) store_s(cf, t, 0, 4 * s + j, 1, 0, false);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[t][0][r] = __builtin_fmaf(cf[r] * dw[j & 1][t][r], dx[j], acc[t][0][r]);
+          for (int r = 0; r < 4; ++r) acc[t][0][r] = __builtin_fmaf(cf[r], pr[t][4 * j + r], acc[t][0][r]);
           asm volatile("" : "+v"(acc[t][0]));
         }
       };
@@ -357,7 +370,6 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
             lo = wf[t][j >> 1][2 * (j & 1)];
             hi = wf[t][j >> 1][2 * (j & 1) + 1];
           }
-          dw[j & 1][t] = *reinterpret_cast<const f32x4*>(scl + (t * 4 + j) * 16 + 4 * g);
           cc[j & 1][t] = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, u32x2{lo, hi}), x[j], corr[j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -366,8 +378,18 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       scale(3);
     } else if constexpr (BLK32) {
       constexpr int NI = 4 * CN;  // i = j * CN + u: block j of the step, column tile u
+      static_assert(CN == 2 || CN % 4 == 0, "four consecutive i share one product instruction");
       f16x8 a[2][WN], x[4];
-      f32x4 dw[2][WN], cc[2][WN], dx[CN];
+      f32x4 cc[2][WN];
+      f32x16 pr[WN];  // d_w * d_x of tiles i & ~3 .. i | 3
+      float pa[WN], pb;
+      auto fetch_scales = [&](int i) {  // of the product instruction's block g: tile i + g
+        const int j = CN == 2 ? i / CN + (g >> 1) : i / CN;
+        const int c = CN == 2 ? 16 * (g & 1) : 16 * (i % CN + g);
+#pragma unroll
+        for (int t = 0; t < WN; ++t) pa[t] = scl[(t * 4 + j) * 16 + r16];
+        pb = reinterpret_cast<const float*>(dxp)[j * L::kDxRow + c + r16];
+      };
       auto fetch = [&](int i) {
         x[i & 3] = *reinterpret_cast<const f16x8*>(b + (i / CN) * L::kPiece + 256 * (i % CN));
       };
@@ -392,7 +414,6 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
             bytes_to_f16(hi, e1, o1);
             a[j & 1][t] = frag(e0, o0, e1, o1);
           }
-          dw[j & 1][t] = *reinterpret_cast<const f32x4*>(scl + (t * 4 + j) * 16 + 4 * g);
         }
       };
       auto scale = [&](int i) {
@@ -402,14 +423,13 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           if (STORE_S && 4 * s + j < nblk && s < s1) store_s(cc[i & 1][t], t, u, 4 * s + j, 1, 0, false);
 #pragma unroll
           for (int r = 0; r < 4; ++r)
-            acc[t][u][r] = __builtin_fmaf(cc[i & 1][t][r] * dw[j & 1][t][r], dx[u][j], acc[t][u][r]);
+            acc[t][u][r] = __builtin_fmaf(cc[i & 1][t][r], pr[t][4 * (i & 3) + r], acc[t][u][r]);
           asm volatile("" : "+v"(acc[t][u]));
         }
       };
       fetch(0);
       fetch(1);
-#pragma unroll
-      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const f32x4*>(dxp + (16 * u + r16) * 16);
+      fetch_scales(0);
       unpack(0);
 #pragma unroll
       for (int i = 0; i < NI; ++i) {
@@ -421,13 +441,20 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           cc[i & 1][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[j & 1][t], x[i & 3], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
         if (i > 0) scale(i - 1);
+        if (i % 4 == 0) {
+#pragma unroll
+          for (int t = 0; t < WN; ++t) pr[t] = outer4(pa[t], pb);
+          if (i + 4 < NI) fetch_scales(i + 4);
+        }
         if (i % CN == CN - 1 && j < 3) unpack(j + 1);
       }
       scale(NI - 1);
     } else if constexpr (TQ2) {
+      constexpr bool OUT4 = CN % 4 == 0;  // d_w * d_x of tiles u & ~3 .. u | 3 from one matrix instruction
       i32x4 a[WN][4], x[2][4], cc[2][WN];
       f32x4 dw[WN];
-      float dx[CN];
+      float dx[CN], pa[WN], pb;
+      f32x16 pr[WN];
       auto fetch = [&](int u) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) x[u & 1][v] = *reinterpret_cast<const i32x4*>(b + v * L::kPiece + 256 * u);
@@ -440,16 +467,24 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
           for (int r = 0; r < 4; ++r) cf[r] = static_cast<float>(cc[u & 1][t][r]);
           if (STORE_S && s < s1) store_s(cf, t, u, s, 1, 0, false);
 #pragma unroll
-          for (int r = 0; r < 4; ++r) acc[t][u][r] = __builtin_fmaf(dx[u] * dw[t][r], cf[r], acc[t][u][r]);
+          for (int r = 0; r < 4; ++r)
+            acc[t][u][r] = __builtin_fmaf(OUT4 ? pr[t][4 * (u & 3) + r] : dx[u] * dw[t][r], cf[r], acc[t][u][r]);
           asm volatile("" : "+v"(acc[t][u]));
         }
       };
       fetch(0);
+      if constexpr (OUT4) {
+        pb = reinterpret_cast<const float*>(dxp)[lane];
+      } else {
 #pragma unroll
-      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+        for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+      }
 #pragma unroll
       for (int t = 0; t < WN; ++t) {
-        dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 16 + 4 * g);
+        if constexpr (OUT4)
+          pa[t] = scl[t * 16 + r16];
+        else
+          dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 16 + 4 * g);
 #pragma unroll
         for (int v = 0; v < 4; ++v)
 #pragma unroll
@@ -467,6 +502,13 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
             cc[u & 1][t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[t][v], x[u & 1][v],
                                                                  v == 0 ? i32x4{0, 0, 0, 0} : cc[u & 1][t], 0, 0, 0);
         if (u > 0) scale(u - 1);
+        if constexpr (OUT4) {
+          if (u % 4 == 0) {
+#pragma unroll
+            for (int t = 0; t < WN; ++t) pr[t] = outer4(pa[t], pb);
+            if (u + 4 < CN) pb = reinterpret_cast<const float*>(dxp)[16 * (u + 4) + lane];
+          }
+        }
       }
       __builtin_amdgcn_sched_barrier(0);
       scale(CN - 1);
@@ -480,7 +522,9 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       f16x8 a[WN][4], x[4];
       f32x4 dw[WN], dm[WN], cc[2][WN], cm[hb ? 2 : 1][WN];
       f16x8 am[WN];
-      float dx[CN];
+      constexpr bool OUT4 = CN % 4 == 0 && hb;  // d * d_x and dmin * d_x of tiles u & ~3 .. u | 3, each one instruction
+      float dx[CN], pa[WN], qa[WN], pb;
+      f32x16 pr[WN], qr[WN];
       const unsigned char* const sp = suml + (((s - s0) >> 1) & 1) * L::kSums + (g & 1) * L::kRow + r16 * 16;
       auto fetch = [&](int i) {
         const int u = i / NF, f = i % NF;
@@ -504,7 +548,8 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const float sd = half[t][u][r] + cc[u & 1][t][r];
-              acc[t][u][r] += __builtin_fmaf(sd, dw[t][r] * dx[u], -cm[u & 1][t][r] * (dm[t][r] * dx[u]));
+              acc[t][u][r] += OUT4 ? __builtin_fmaf(sd, pr[t][4 * (u & 3) + r], -cm[u & 1][t][r] * qr[t][4 * (u & 3) + r])
+                                   : __builtin_fmaf(sd, dw[t][r] * dx[u], -cm[u & 1][t][r] * (dm[t][r] * dx[u]));
             }
             asm volatile("" : "+v"(acc[t][u]));  // as above
           }
@@ -512,12 +557,21 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       };
       fetch(0);
       fetch(1);
+      if constexpr (OUT4) {
+        pb = reinterpret_cast<const float*>(dxp)[lane];
+      } else if constexpr (hb) {
 #pragma unroll
-      for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+        for (int u = 0; u < CN; ++u) dx[u] = *reinterpret_cast<const float*>(dxp + (16 * u + r16) * 4);
+      }
 #pragma unroll
       for (int t = 0; t < WN; ++t) {
-        if constexpr (hb) dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 4 * g);
-        if constexpr (hb) dm[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 16 + 4 * g);
+        if constexpr (OUT4) {
+          pa[t] = scl[t * 32 + r16];
+          qa[t] = scl[t * 32 + 16 + r16];
+        } else if constexpr (hb) {
+          dw[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 4 * g);
+          dm[t] = *reinterpret_cast<const f32x4*>(scl + t * 32 + 16 + 4 * g);
+        }
         const u32x4 e = *reinterpret_cast<const u32x4*>(scl + WN * 32 + t * 64 + r16 * 4);
         const unsigned sc = hb ? (e[3] & 0x0F0F0F0Fu) | ((e[1] >> 2) & 0x30303030u) : e[1] & 0x3F3F3F3Fu;
 #pragma unroll
@@ -559,6 +613,16 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
         }
         __builtin_amdgcn_sched_barrier(0);
         if (f == 1 && u > 0) scale(u - 1);
+        if constexpr (OUT4) {
+          if (f == 1 && u % 4 == 0) {
+#pragma unroll
+            for (int t = 0; t < WN; ++t) {
+              pr[t] = outer4(pa[t], pb);
+              qr[t] = outer4(qa[t], pb);
+            }
+            if (u + 4 < CN) pb = reinterpret_cast<const float*>(dxp)[16 * (u + 4) + lane];
+          }
+        }
       }
       scale(CN - 1);
     }
@@ -703,22 +767,27 @@ hipError_t launch_fmt(const GemmCall& c, const TilePlan& p, hipStream_t stream) 
       default: return hipErrorInvalidConfiguration;
     }
   }
-#define KOMP_TILE_PLAN(RW, WN, CN, WK) \
-  if (p.rw == RW && p.wn == WN && p.cn == CN && p.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, false>(c, stream);
-  KOMP_TILE_PLAN(1, 1, 1, 8)
-  KOMP_TILE_PLAN(1, 2, 1, 8)
-  KOMP_TILE_PLAN(1, 2, 1, 4)
-  KOMP_TILE_PLAN(2, 1, 2, 4)
-  KOMP_TILE_PLAN(2, 2, 2, 4)
-  KOMP_TILE_PLAN(2, 1, 4, 4)
-  KOMP_TILE_PLAN(4, 1, 4, 2)
-  KOMP_TILE_PLAN(4, 1, 8, 2)
-  KOMP_TILE_PLAN(4, 2, 4, 1)
-  KOMP_TILE_PLAN(8, 1, 8, 1)
-  if constexpr (FMT != FMT_Q4_K) {  // Q4_K's waves also hold a block's first half of every output: too many registers
-    KOMP_TILE_PLAN(4, 2, 8, 1)
-    KOMP_TILE_PLAN(4, 2, 8, 2)
-  }
+#define KOMP_TILE_PLAN(ON, RW, WN, CN, WK)                                  \
+  if constexpr (ON)                                                         \
+    if (p.rw == RW && p.wn == WN && p.cn == CN && p.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, false>(c, stream);
+  constexpr bool q4 = FMT == FMT_Q4_0 || FMT == FMT_IQ4_NL, tq2 = FMT == FMT_TQ2_0, q8 = FMT == FMT_Q8_0, qk = FMT == FMT_Q4_K;
+  KOMP_TILE_PLAN(true, 1, 1, 1, 8)
+  KOMP_TILE_PLAN(true, 1, 2, 1, 8)
+  KOMP_TILE_PLAN(true, 1, 2, 1, 4)
+  KOMP_TILE_PLAN(q4 || tq2, 1, 1, 1, 4)
+  KOMP_TILE_PLAN(tq2, 2, 1, 1, 4)
+  KOMP_TILE_PLAN(q4 || tq2, 2, 2, 1, 4)
+  KOMP_TILE_PLAN(!q8, 2, 1, 2, 4)
+  KOMP_TILE_PLAN(true, 2, 2, 2, 4)
+  KOMP_TILE_PLAN(qk, 2, 1, 4, 4)
+  KOMP_TILE_PLAN(true, 4, 1, 4, 2)
+  KOMP_TILE_PLAN(q4 || tq2, 4, 2, 4, 2)
+  KOMP_TILE_PLAN(q4 || q8, 4, 2, 4, 1)
+  KOMP_TILE_PLAN(qk, 4, 1, 8, 2)
+  KOMP_TILE_PLAN(q4 || tq2, 4, 2, 8, 1)
+  KOMP_TILE_PLAN(q4 || q8, 4, 2, 8, 2)
+  KOMP_TILE_PLAN(!q4, 8, 1, 8, 1)
+  KOMP_TILE_PLAN(!qk, 8, 2, 8, 1)  // (Q4_K's waves also hold a block's first half of every output: too many registers)
 #undef KOMP_TILE_PLAN
   return hipErrorInvalidConfiguration;
 }

@@ -40,10 +40,24 @@ PLANS = [(64, 5), (4331, 5), (8400, 9), (1420, 33), (4331, 20), (8400, 20), (234
 @pytest.mark.parametrize("shape", range(len(PLANS)))
 def test_every_plan(fmt, shape):
     n, m = PLANS[shape]
+    check_large(fmt, n, 1536 if O.FORMATS[fmt]["block"] == 256 else 736, m, shape)
+
+
+# the plans of gemm_tile_plan that the shapes above do not take, on a 256-CU device
+MORE = [("q4_0", 28700, 1056, 66), ("iq4_nl", 4099, 1056, 5), ("q4_0", 12330, 672, 17), ("q4_0", 16500, 672, 1100),
+        ("tq2_0", 70, 2304, 5), ("tq2_0", 4099, 2304, 5), ("tq2_0", 28700, 1536, 260), ("tq2_0", 28700, 1536, 5),
+        ("q8_0", 20000, 672, 768), ("q8_0", 12330, 672, 17), ("q4_k", 4099, 2304, 9), ("q4_k", 8211, 1792, 17)]
+
+
+@pytest.mark.parametrize("fmt,n,k,m", MORE)
+def test_more_plans(fmt, n, k, m):
+    check_large(fmt, n, k, m, n + m)
+
+
+def check_large(fmt, n, k, m, seed):
     blk = O.FORMATS[fmt]["block"]
-    k = 1536 if blk == 256 else 736
     nb = k // blk
-    rng = np.random.default_rng(shape)
+    rng = np.random.default_rng(seed)
     W = O.weights(fmt, rng, n, k)
     wq, ws = host.split(fmt, W, n, k)
     x = O.activations(rng, k, m, block=O.ACT_BLOCK[O.FORMATS[fmt]["act"]])
