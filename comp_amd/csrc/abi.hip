@@ -409,7 +409,8 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 //     (4096 x 14336 13.3 us against 16.3, 28672 x 4096 at 5 columns 24.8 against 25.3); up to 16 over at most 2 row tiles a
 //     CU where rows are long or few (2560 x 6912 at 16 columns 9.2 against 9.8, 127 x 2816 5.1 against 6.1; 4096 x 4096 7.6
 //     against 7.0 goes to the tile); up to 32 where two column groups are just past a workgroup a CU (2560 x 6912 at 24
-//     columns 11.6 against 12.8).
+//     columns 11.6 against 12.8); and 49-64 columns over about one row tile a CU, where komp_gemm_plan's answer of one group
+//     of 64 columns is part of the interface (the tile's two groups would take 4096 x 14336 in 31.5 us against 42).
 //
 // The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
@@ -452,7 +453,8 @@ bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePl
   if (steps <= 4 || n < 1) return false;
   if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
   if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus && (nblk > 24 || n <= cus)) ||
-                          (m <= 32 && n > 8 * cus && n <= 12 * cus)))
+                          (m <= 32 && n > 8 * cus && n <= 12 * cus) ||
+                          (m > 48 && m <= 64 && n > 8 * cus && n <= 16 * cus)))
     return false;
   const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : fmt == FMT_Q4_K ? 3 : 0;
   double best = -1;
