@@ -38,8 +38,9 @@
 // crossed with g put those on different banks.  (Padding every unit row by 16 bytes instead left the reads with 42% of
 // their LDS cycles in conflicts.)
 //
-// What it reaches: Q4_0 14336 x 4096 at 512 columns 105 us, of which the VALU's issue slots (matrix instructions
-// included) are about 95 at the 7/8 of its CUs that the tiles fill evenly; TQ2_0 6912 x 2560 at 2048 columns 64 us.
+// What it reaches: Q4_0 14336 x 4096 at 512 columns 105 us, of which VALU issue (4 clocks an instruction, 8 a matrix
+// instruction, 28 an outer product) is 77 on the CUs that have a workgroup (224 of 256); Q4_K 4096 x 14336 at 1001 columns
+// 188 a call, issue 116 and LDS half the time; TQ2_0 6912 x 2560 at 2048 columns 64.
 #pragma once
 
 #include <hip/hip_ext.h>
