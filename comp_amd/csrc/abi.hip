@@ -405,6 +405,11 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 // 512 columns 385 -> 105, Q8_0 14336 x 4096 at 16 columns 24.3 -> 14.1, TQ2_0 6912 x 2560 at 8 columns 6.3 -> 4.7, at 2048
 // columns 326 -> 61, Q4_K 4096 x 14336 at 1001 columns 561 -> 181.  gemm.hip's kernel keeps
 //   rows of at most 4 K steps, which are over before the tile's staging pays;
+//   up to 8 columns over at most a row a CU (Q4_0 127 x 4192 5.1 us against 5.3, TQ2_0 127 x 2816 3.8 against 4.1; Q8_0 is
+//     as fast on the tile) and, of the 4-bit formats' long rows, over one row tile a CU (Q4_0 4096 x 14336 at 4 columns
+//     12.7 against 13.6; 4096 x 4096 5.7 against 5.5);
+//   Q8_0 up to 16 columns just past one row tile a CU (4097 x 4192 at 8 columns 9.7 against 11.2; 6144 x 4096 11.9 against
+//     9.1);
 //   Q4_K's few columns, whose scale products the tile multiplies into the weights once per column group: up to 8 columns
 //     (4096 x 14336 13.3 us against 16.3, 28672 x 4096 at 5 columns 24.8 against 25.3); up to 16 over at most 2 row tiles a
 //     CU where rows are long or few (2560 x 6912 at 16 columns 9.2 against 9.8, 127 x 2816 5.1 against 6.1; 4096 x 4096 7.6
@@ -450,12 +455,15 @@ bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePl
   const int64_t nblk = k / fmt_info(fmt).block;
   const int64_t steps = fmt == FMT_Q4_K ? 2 * nblk : fmt == FMT_TQ2_0 ? nblk : (nblk + 3) / 4;
   const int64_t cus = device_cus();
+  const bool blk32 = fmt_info(fmt).block == 32;
   if (steps <= 4 || n < 1) return false;
   if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
   if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus && (nblk > 24 || n <= cus)) ||
                           (m <= 32 && n > 8 * cus && n <= 12 * cus) ||
                           (m > 48 && m <= 64 && n > 8 * cus && n <= 16 * cus)))
     return false;
+  if (m <= 8 && ((fmt != FMT_Q8_0 && n <= cus) || (blk32 && fmt != FMT_Q8_0 && nblk > 256 && n <= 16 * cus))) return false;
+  if (m <= 16 && fmt == FMT_Q8_0 && n > 16 * cus && n <= 20 * cus) return false;
   const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : fmt == FMT_Q4_K ? 3 : 0;
   double best = -1;
   for (const TileCost& t : kTileCosts) {

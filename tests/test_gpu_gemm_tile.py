@@ -45,7 +45,7 @@ def test_every_plan(fmt, shape):
 
 # the plans of gemm_tile_plan that the shapes above do not take, on a 256-CU device
 MORE = [("q4_0", 28700, 1056, 66), ("iq4_nl", 4099, 1056, 5), ("q4_0", 12330, 672, 17), ("q4_0", 16500, 672, 1100),
-        ("tq2_0", 70, 2304, 5), ("tq2_0", 4099, 2304, 5), ("tq2_0", 28700, 1536, 260), ("tq2_0", 28700, 1536, 5),
+        ("tq2_0", 70, 2304, 9), ("tq2_0", 4099, 2304, 5), ("tq2_0", 28700, 1536, 260), ("tq2_0", 28700, 1536, 5),
         ("q8_0", 20000, 672, 768), ("q8_0", 12330, 672, 17), ("q4_k", 4099, 2304, 9), ("q4_k", 8211, 1792, 17)]
 
 
