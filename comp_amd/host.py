@@ -170,8 +170,9 @@ def ctypes_stream(dev):
 # An eager call is mostly host time (15 us a call against 3 us of kernel at the decode shapes): its checks are one chain
 # of cheap attribute reads that must imply the full check, which runs, and names the fault, when any of them fails; the
 # current stream's handle comes without a Stream object (2.1 us), and the device is switched only if it is another one.
-_raw_stream = torch._C._cuda_getCurrentRawStream
-_current_device = torch._C._cuda_getDevice
+# (A torch without GPU support has neither function; there, nothing launches.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", ctypes_stream)
+_current_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)
 _Tensor, _U8, _I16, _I8, _F32 = torch.Tensor, torch.uint8, torch.int16, torch.int8, torch.float32
 
 
