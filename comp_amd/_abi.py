@@ -116,15 +116,9 @@ def check(status, what):
     raise KompError(msg)
 
 
-_entries = {}
-
-
 def entry(name):
-    """An ABI function of the loaded library (looked up once)."""
-    fn = _entries.get(name)
-    if fn is None:
-        fn = _entries[name] = getattr(lib(), name)
-    return fn
+    """An ABI function of the loaded library (which keeps it as an attribute after the first look)."""
+    return getattr(_lib or lib(), name)
 
 
 def call(name, *args):
