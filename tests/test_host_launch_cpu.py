@@ -1,12 +1,14 @@
-"""How comp_amd.host reaches the library, without a GPU: what importing it needs of torch, and which
-library its calls go to."""
+"""How comp_amd.host reaches the library, without a GPU: what importing it needs of torch, which
+library its calls go to, and what they hand over and return."""
 
 import os
 import subprocess
 import sys
 import types
 
-from comp_amd import _abi
+import torch
+
+from comp_amd import _abi, host
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -34,3 +36,26 @@ def test_calls_go_to_the_library_that_is_loaded_now(monkeypatch):
         _abi.call("komp_quant_q8_0")
         assert _abi.entry("komp_quant_q8_0")() == 0
     assert got == [1, 1, 2, 2]
+
+
+class DeviceLike(torch.Tensor):
+    """A tensor subclass that says it is on a device (its memory is the host's; nothing launches)."""
+
+    is_cuda = True
+
+
+def test_outputs_are_plain_tensors_whatever_the_inputs_type(monkeypatch):
+    """As torch.empty gives them: a subclass of the input's would run its own code on every later use of a plane."""
+    monkeypatch.setattr(host, "_launch", lambda name, *a: None)
+    monkeypatch.setattr(host, "_check_gemv", lambda *a: (2, 4))
+    monkeypatch.setattr(host, "_weights_fit", lambda *a: True)
+    like = lambda *shape, dtype=torch.float32: torch.zeros(shape, dtype=dtype).as_subclass(DeviceLike)  # noqa: E731
+    x, w = like(2, 1024), like(8, 512, dtype=torch.uint8)
+    q = (*host.quantize("q4_0", x), *host.quantize("tq2_0", x, bsums=True))
+    xq, xd = like(2, 1024, dtype=torch.int8), like(2, 32)
+    y = [f("q4_0", w, w, xq, xd, 8, 1024)[0] for f in (host.gemv, host.gemm)] + [host.gemv_f32("q4_0", w, w, x, 8, 1024)[0]]
+    assert [type(t) for t in (*q, *y)] == [torch.Tensor] * 8
+    assert [(t.shape, t.dtype) for t in y] == [((2, 8), torch.float32)] * 3
+    assert [(tuple(t.shape), t.dtype) for t in q] == [
+        ((2, 1024), torch.int8), ((2, 32), torch.float32),
+        ((2, 1024), torch.int8), ((2, 4), torch.float32), ((2, 64), torch.int16)]  # fmt: skip
