@@ -62,6 +62,7 @@ SIGNATURES = {
     "komp_q4_0_gemm": (_INT, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "komp_tq2_0_gemm": (_INT, [_P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _P]),
     "komp_gemm_plan": (_INT, [_INT, _I64, _I64, _I64, _I64, _P, _P, _P]),
+    "komp_gemm_launch": (_INT, [_INT, _INT, _I64, _I64, _I64, _I64, _P, _P, _P, _P, _P, _P]),
     "komp_gemv_mfma_plan": (_INT, [_INT, _INT, _INT, _I64, _I64, _I64, _I64, _P, _P]),
     "komp_q4_0_split": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
     "komp_tq2_0_split": (_INT, [_P, _P, _P, _I64, _I64, _I64, _P]),
@@ -142,6 +143,14 @@ def gemm_plan(fmt_id, m, n, k, sw):
     v = [ctypes.c_int(0) for _ in range(3)]
     st = lib().komp_gemm_plan(fmt_id, m, n, k, sw, *(ctypes.byref(x) for x in v))
     return tuple(x.value for x in v) if st == 0 else None
+
+
+def gemm_launch(fmt_id, m, n, k, sw, store_s=False):
+    """(tiled, K groups, row groups, row tiles, column tiles, column groups) of the launch komp_*_gemm makes, or None past
+    its limits."""
+    v = [ctypes.c_int(0) for _ in range(6)]
+    st = lib().komp_gemm_launch(fmt_id, int(store_s), m, n, k, sw, *(ctypes.byref(x) for x in v))
+    return (bool(v[0].value), *(x.value for x in v[1:])) if st == 0 else None
 
 
 def gemv_mfma_plan(fmt_id, fused, mode, m, n, k, sw):

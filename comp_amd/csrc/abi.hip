@@ -326,7 +326,7 @@ GemvPlan knob_plan(int fmt, int block_n, int nb, int num_warps) {
 // are as fast or faster (TQ2_0 6912 x 2560: 5.6 against 5.8 us, 2560 x 6912: 5.7 against 5.2, 32768 x 8192: 22.5
 // against 23.9; Q4_0 4096 x 14336: 9.9 against 13.9).
 constexpr int64_t kGemmMinM = 4;
-constexpr int64_t kGemmMaxCols = int64_t{1} << 20;  // columns per GEMM launch (grid.y = columns / 64 at most 16384)
+constexpr int64_t kGemmMaxCols = 16 * 65535;  // columns per GEMM launch: at most 65535 column groups (grid.y) of 16
 
 // The GEMM's plan for m columns (one launch) and n rows.  Columns go in groups of at most 64 (4 tiles of 16), split
 // evenly.  The waves of a workgroup split K (wk) and rows (wr) by how many 16-row tiles each CU gets (r, counting
@@ -450,7 +450,7 @@ constexpr TileCost kTileCosts[] = {
 };
 
 // False when the call stays on gemm.hip's kernel: by the rules above, or past the tile's 32-bit buffer offsets (128 rows
-// of SW bytes, 128 columns of K) or the grid's column groups.
+// of SW bytes, 128 columns of K).
 bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePlan* p) {
   const int64_t nblk = k / fmt_info(fmt).block;
   const int64_t steps = fmt == FMT_Q4_K ? 2 * nblk : fmt == FMT_TQ2_0 ? nblk : (nblk + 3) / 4;
@@ -469,7 +469,7 @@ bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePl
   for (const TileCost& t : kTileCosts) {
     const auto& f = t.f[row];
     const int64_t groups = (m + 16 * t.p.cn - 1) / (16 * t.p.cn);
-    if (f.slots == 0 || groups > 65535) continue;
+    if (f.slots == 0) continue;
     const int64_t wgs = (n + 16 * t.p.wn * t.p.rw - 1) / (16 * t.p.wn * t.p.rw) * groups;
     const int64_t load = (wgs + cus - 1) / cus;  // workgroups on the fullest CU
     const int64_t per = fmt == FMT_Q4_K ? 2 * ((nblk + t.p.wk - 1) / t.p.wk) : (steps + t.p.wk - 1) / t.p.wk;
@@ -888,6 +888,29 @@ int komp_gemm_plan(int fmt, int64_t M, int64_t N, int64_t K, int64_t SW, int* ro
   if (rows_per_wg != nullptr) *rows_per_wg = 16 * p.wn * p.wr;
   if (cols_per_wg != nullptr) *cols_per_wg = 16 * p.cn;
   if (waves != nullptr) *waves = p.wk * p.wr;
+  return KOMP_OK;
+}
+
+int komp_gemm_launch(int fmt, int store_s, int64_t M, int64_t N, int64_t K, int64_t SW, int* tiled, int* k_groups,
+                     int* row_groups, int* row_tiles, int* col_tiles, int* col_groups) {
+  if (fmt < FMT_Q4_0 || fmt > FMT_Q4_K) return fail(KOMP_EINVAL, "komp_gemm_launch: fmt=%d", fmt);
+  if (M < 1 || N < 1 || K < 0 || SW < 0) return fail(KOMP_EINVAL, "komp_gemm_launch: bad argument");
+  const int64_t m = M < kGemmMaxCols ? M : kGemmMaxCols;
+  GemmPlan p;
+  if (!gemm_plan(fmt, m, N, K, SW, &p))
+    return fail(KOMP_EINVAL, "komp_gemm_launch: K=%lld / SW=%lld past the GEMM's limits", (long long)K, (long long)SW);
+  TilePlan t;
+  const bool on = gemm_tile_plan(fmt, m, N, K, SW, &t);
+  if (on) {
+    if (store_s) t = tile_plan_with_s(t);
+    p = GemmPlan{t.wk, t.rw, t.wn, t.cn, 1};
+  }
+  if (tiled != nullptr) *tiled = on;
+  if (k_groups != nullptr) *k_groups = p.wk;
+  if (row_groups != nullptr) *row_groups = p.wr;
+  if (row_tiles != nullptr) *row_tiles = p.wn;
+  if (col_tiles != nullptr) *col_tiles = p.cn;
+  if (col_groups != nullptr) *col_groups = static_cast<int>((m + 16 * p.cn - 1) / (16 * p.cn));
   return KOMP_OK;
 }
 

@@ -755,18 +755,19 @@ hipError_t launch_plan(const GemmCall& c, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// The instantiated plans (gemm_tile_plan in abi.hip picks one).  With S, a smaller tile with the same K split runs: its
-// sums run in the same order, so Y is the same bit for bit, and the scattered stores' addresses leave no room for more.
+// The instantiated plans (gemm_tile_plan in abi.hip picks one; with S, tile_plan_with_s of it).
 template <int FMT>
 hipError_t launch_fmt(const GemmCall& c, const TilePlan& p, hipStream_t stream) {
   if (c.s != nullptr) {
-    switch (p.wk) {
-      case 1: return launch_plan<FMT, 2, 1, 2, 1, true>(c, stream);
-      case 2: return launch_plan<FMT, 2, 1, 2, 2, true>(c, stream);
-      case 4: return launch_plan<FMT, 1, 1, 1, 4, true>(c, stream);
-      case 8: return launch_plan<FMT, 1, 1, 1, 8, true>(c, stream);
-      default: return hipErrorInvalidConfiguration;
-    }
+    const TilePlan q = tile_plan_with_s(p);
+#define KOMP_TILE_PLAN_S(RW, WN, CN, WK) \
+  if (q.rw == RW && q.wn == WN && q.cn == CN && q.wk == WK) return launch_plan<FMT, RW, WN, CN, WK, true>(c, stream);
+    KOMP_TILE_PLAN_S(2, 1, 2, 1)
+    KOMP_TILE_PLAN_S(2, 1, 2, 2)
+    KOMP_TILE_PLAN_S(1, 1, 1, 4)
+    KOMP_TILE_PLAN_S(1, 1, 1, 8)
+#undef KOMP_TILE_PLAN_S
+    return hipErrorInvalidConfiguration;
   }
 #define KOMP_TILE_PLAN(ON, RW, WN, CN, WK)                                  \
   if constexpr (ON)                                                         \

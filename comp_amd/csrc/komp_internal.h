@@ -113,6 +113,12 @@ struct TilePlan {
   int wk;
 };
 
+// The tile that runs when S is written as well: a smaller one with the same K split, so its sums run in the same order
+// and Y is the same bit for bit (the scattered stores' addresses leave no registers for more).
+constexpr TilePlan tile_plan_with_s(const TilePlan& p) {
+  return p.wk <= 2 ? TilePlan{2, 1, 2, p.wk} : TilePlan{1, 1, 1, p.wk};
+}
+
 struct GemmCall {
   int fmt;
   const uint8_t* wq;

@@ -197,6 +197,13 @@ int komp_tq2_0_gemm(const uint8_t* WQ, const int16_t* WS, const int8_t* XQ, cons
 int komp_gemm_plan(int fmt, int64_t M, int64_t N, int64_t K, int64_t SW, int* rows_per_wg, int* cols_per_wg,
                    int* waves);
 
+/* The first launch that komp_*_gemm makes for a shape, in full: tiled 1 for the tiled kernel, 0 for the batched one, the
+ * workgroup's K groups x row groups of waves, 16-row tiles a row group, 16-column tiles, and the launch's column groups
+ * (at most 65535; more columns are further launches).  store_s: of a call that writes S (for the tiled kernel).  NULL
+ * outputs are skipped.  Returns KOMP_EINVAL when the shape is past the kernel's limits.  No reference counterpart. */
+int komp_gemm_launch(int fmt, int store_s, int64_t M, int64_t N, int64_t K, int64_t SW, int* tiled, int* k_groups,
+                     int* row_groups, int* row_tiles, int* col_tiles, int* col_groups);
+
 /* Whether komp_tq2_0_gemv with block_n == 0 runs the matrix-core GEMV for this call (fused 0 / 1, mode as the GEMVs):
  * TQ2_0, KOMP_MODE_DP4A, 3 columns, more than 8 rows a CU, rows of at most 64 blocks, SW a multiple of 16, q8_K
  * activations in (f32 in: from 4 row tiles a CU on).  Returns 1 and its workgroup's rows (spread evenly over the

@@ -1,0 +1,33 @@
+"""Which matrix-core GEMM launch a call makes (the library's plan query; no GPU needed)."""
+
+import pytest
+
+from comp_amd import _abi, host
+
+FMTS = sorted(host.FMT_ID)
+
+
+def launch(fmt, m, n, k, store_s=False):
+    f = host.FORMATS[fmt]
+    return _abi.gemm_launch(host.FMT_ID[fmt], m, n, k, k // f["block"] * f["qbytes"], store_s)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_column_groups_fit_the_grid(fmt):
+    """Whatever the plan's column tiles, and with S the smaller ones of the launch that writes it."""
+    for m in (1, 16 * 65535, 1 << 20, 1 << 24):
+        for n in (1, 100, 3000):
+            for k in (1280, 2048, 4096, 8192):
+                for store_s in (False, True):
+                    _, _, _, _, col_tiles, col_groups = launch(fmt, m, n, k, store_s)
+                    assert 1 <= col_groups <= 65535 and 16 * col_tiles * col_groups >= min(m, 16 * 65535)
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_s_keeps_the_k_split(fmt):
+    """Y is the same bit for bit with and without S: both launches split K alike."""
+    for m in (4, 20, 60, 300, 2000):
+        for n in (64, 2000, 9000, 40000):
+            for k in (1280, 4096, 14336):
+                a, b = launch(fmt, m, n, k), launch(fmt, m, n, k, True)
+                assert a[0] == b[0] and a[1] == b[1]
