@@ -137,7 +137,8 @@ gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __restrict
   const int m0 = blockIdx.y * (16 * CN);
   const int rows = max(0, min(16 * WN, N - nw));  // valid rows of this wave's tiles, valid columns of the workgroup
   const int cols = min(16 * CN, M - m0);
-  const auto wq = rsrc(WQ + nw * SW, rows * SW);
+  // to the end of the last row's blocks, not of its stride: the plane may be a view of some of a larger one's columns
+  const auto wq = rsrc(WQ + nw * SW, (rows - 1) * SW + static_cast<int64_t>(nblk) * fmt_info(FMT).qbytes);
   const auto xq = rsrc(XQ + static_cast<int64_t>(m0) * K, static_cast<int64_t>(cols) * K);
   const auto xd = rsrc(XD + static_cast<int64_t>(m0) * nblk, static_cast<int64_t>(cols) * nblk * 4);
 
@@ -145,7 +146,7 @@ gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __restrict
   // its per-lane offset (plus an immediate), which the range check covers; the buffer instruction's scalar offset is
   // always 0.  A step past the wave's last adds kOob instead (every per-lane offset is below 2^31, so the sum does
   // not wrap), which makes all of its loads return zeros without touching memory.  In a partial last Q4_0 step the
-  // lanes of blocks past K read the next row's (column's) first bytes, or zeros past the tensor's end; those blocks
+  // lanes of blocks past K read the next row's (column's) first bytes, or zeros past the tile's last one; those blocks
   // are skipped when the step is computed.
   unsigned va[WN];
 #pragma unroll

@@ -168,7 +168,8 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   unsigned char* const wl = lds + WK * L::kGroup + wave * L::wave(WN);
   float* const scl = reinterpret_cast<float*>(wl + L::weights(WN));
 
-  const auto wq = rsrc(WQ + nw * SW, rows * SW);
+  // to the end of the last row's blocks, not of its stride: the plane may be a view of some of a larger one's columns
+  const auto wq = rsrc(WQ + nw * SW, (rows - 1) * SW + static_cast<int64_t>(nblk) * fmt_info(FMT).qbytes);
   const auto ws = rsrc(WS + static_cast<int64_t>(nw) * nblk * (QK ? 8 : 1),
                        static_cast<int64_t>(rows) * nblk * (QK ? 16 : 2));
   const auto xq = rsrc(XQ + static_cast<int64_t>(m0) * K, static_cast<int64_t>(cols) * K);
