@@ -141,7 +141,8 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
   constexpr int BI = COLS * PC / T;    // staging items a thread
   static_assert(BI * T == COLS * PC, "the threads split the staged columns evenly");
   extern __shared__ __align__(16) unsigned char lds[];
-  // kBias in a VGPR, so that masking a nibble pair and putting the bias on is one v_and_or_b32 (which takes one literal)
+  // the bias (1024 in both f16) in a VGPR, so that masking a nibble pair and putting it on is one v_and_or_b32 (which
+  // takes one literal)
   unsigned bias;
   asm("v_mov_b32 %0, 0x64006400" : "=v"(bias));
   const int lane = threadIdx.x & 63;
@@ -334,7 +335,8 @@ tile_gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __res
       // tile and block against 3 and 4 conversions), and so would the activations'
       long x[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) x[j] = *reinterpret_cast<const long*>(b + j * L::kPiece);
+      for (int j = 0; j < 4; ++j)  // (vector types may alias the staged dwords; long may not)
+        x[j] = __builtin_bit_cast(long, *reinterpret_cast<const u32x2*>(b + j * L::kPiece));
       i32x4 corr[4], cc[2][WN];
       f32x16 pr[WN];  // d_w * d_x: instruction block j is the step's block j
       const float dx = reinterpret_cast<const float*>(dxp)[g * L::kDxRow + r16];
