@@ -137,8 +137,9 @@ gemm_kernel(int N, int M, int K, int nblk, int64_t SW, const uint8_t* __restrict
   const int m0 = blockIdx.y * (16 * CN);
   const int rows = max(0, min(16 * WN, N - nw));  // valid rows of this wave's tiles, valid columns of the workgroup
   const int cols = min(16 * CN, M - m0);
-  // to the end of the last row's blocks, not of its stride: the plane may be a view of some of a larger one's columns
-  const auto wq = rsrc(WQ + nw * SW, (rows - 1) * SW + static_cast<int64_t>(nblk) * fmt_info(FMT).qbytes);
+  // The range of 32-value blocks, whose last K step may be partial, ends with the last row's blocks, not its stride: the
+  // plane may be a view of some of a larger one's columns
+  const auto wq = rsrc(WQ + nw * SW, BLK32 ? (rows - 1) * SW + static_cast<int64_t>(nblk) * (Q8 ? 32 : 16) : rows * SW);
   const auto xq = rsrc(XQ + static_cast<int64_t>(m0) * K, static_cast<int64_t>(cols) * K);
   const auto xd = rsrc(XD + static_cast<int64_t>(m0) * nblk, static_cast<int64_t>(cols) * nblk * 4);
 

@@ -21,7 +21,7 @@ struct FmtInfo {
   int soff;
   int sbytes;
 };
-constexpr FmtInfo fmt_info(int fmt) {
+inline FmtInfo fmt_info(int fmt) {
   switch (fmt) {
     case FMT_TQ2_0: return FmtInfo{256, 66, 64, 0, 64, 2};
     case FMT_Q8_0: return FmtInfo{32, 34, 32, 2, 0, 2};
