@@ -468,10 +468,13 @@ bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePl
   double best = -1;
   for (const TileCost& t : kTileCosts) {
     const auto& f = t.f[row];
-    const int64_t groups = (m + 16 * t.p.cn - 1) / (16 * t.p.cn);
     if (f.slots == 0) continue;
-    const int64_t wgs = (n + 16 * t.p.wn * t.p.rw - 1) / (16 * t.p.wn * t.p.rw) * groups;
-    const int64_t load = (wgs + cus - 1) / cus;  // workgroups on the fullest CU
+    const int64_t gx = (n + 16 * t.p.wn * t.p.rw - 1) / (16 * t.p.wn * t.p.rw);
+    const int64_t gy = (m + 16 * t.p.cn - 1) / (16 * t.p.cn);
+    // workgroups on the fullest CU: a row group's column groups run on one of the 8 XCDs.  (Counted over all CUs at once,
+    // 5200 rows at 65-96 columns went to plans that leave two XCDs 33 workgroups for 32 CUs: 8192 values of K at 65
+    // columns Q4_0 49.1 -> 34.0 us, TQ2_0 at 4096 14.9 -> 9.7.)
+    const int64_t load = ((gx + 7) / 8 * gy * 8 + cus - 1) / cus;
     const int64_t per = fmt == FMT_Q4_K ? 2 * ((nblk + t.p.wk - 1) / t.p.wk) : (steps + t.p.wk - 1) / t.p.wk;
     const double rounds = load > f.slots ? static_cast<double>(load) / f.slots : 1.0;
     const double us = per * (f.a * rounds + f.b * static_cast<double>(load));

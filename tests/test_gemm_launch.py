@@ -31,3 +31,13 @@ def test_s_keeps_the_k_split(fmt):
             for k in (1280, 4096, 14336):
                 a, b = launch(fmt, m, n, k), launch(fmt, m, n, k, True)
                 assert a[0] == b[0] and a[1] == b[1]
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+@pytest.mark.parametrize("m", [65, 80, 96])
+def test_one_round_of_workgroups_fits_every_xcd(fmt, m):
+    """5200 rows by a few column groups: a row group's column groups share one of the 8 XCDs, so a plan of at most a
+    workgroup a CU in all must not leave an XCD more of them than its 32 CUs (a second round there costs 45-65%)."""
+    _, k_groups, row_groups, row_tiles, _, col_groups = launch(fmt, m, 5200, 8192)
+    groups = -(-5200 // (16 * row_groups * row_tiles))
+    assert groups * col_groups > 256 or -(-groups // 8) * col_groups <= 32
