@@ -421,7 +421,9 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
 // launch has 3 us besides.  The constants are fitted to 12 column counts from 5 to 2048 over 8 or 9 shapes a format (127 to
 // 28672 rows); the plan they pick is within 1-2.5% of the fastest of all 22 measured ones in the geometric mean, and a format
-// leaves out the plans that this does not need.
+// leaves out the plans that this does not need.  Q4_K's are fitted to 1732 shapes (768 to 28672 rows, 1280 to 14336 values of
+// K, 4 to 512 columns; 0.1% from the fastest): with one constant a plan, short rows went to workgroups of 16 rows and 8 K
+// groups, 9216 x 1536 at 16 columns 12.2 us against 8.2 now.
 struct TileCost {
   TilePlan p;
   struct {
@@ -430,22 +432,22 @@ struct TileCost {
   } f[4];  // Q4_0 and IQ4_NL, TQ2_0, Q8_0, Q4_K
 };
 constexpr TileCost kTileCosts[] = {
-    {{1, 1, 1, 8}, {{2, 0.f, 0.60f}, {1, 0.f, 0.78f}, {1, 0.f, 0.80f}, {1, 0.f, 0.88f}}},
-    {{1, 2, 1, 8}, {{2, 0.f, 0.82f}, {1, 0.f, 1.11f}, {3, 0.f, 1.08f}, {1, 0.f, 1.40f}}},
-    {{1, 2, 1, 4}, {{4, 0.11f, 0.39f}, {2, 0.20f, 0.39f}, {2, 0.10f, 0.47f}, {3, 0.33f, 0.50f}}},
+    {{1, 1, 1, 8}, {{2, 0.f, 0.60f}, {1, 0.f, 0.78f}, {1, 0.f, 0.80f}, {4, 0.71f, 0.86f}}},
+    {{1, 2, 1, 8}, {{2, 0.f, 0.82f}, {1, 0.f, 1.11f}, {3, 0.f, 1.08f}, {3, 0.29f, 1.68f}}},
+    {{1, 2, 1, 4}, {{4, 0.11f, 0.39f}, {2, 0.20f, 0.39f}, {2, 0.10f, 0.47f}, {3, 0.70f, 0.45f}}},
     {{1, 1, 1, 4}, {{2, 0.16f, 0.18f}, {2, 0.24f, 0.21f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
     {{2, 1, 1, 4}, {{0, 0.f, 0.f}, {2, 0.11f, 0.45f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
     {{2, 2, 1, 4}, {{2, 0.21f, 0.69f}, {2, 0.03f, 0.95f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
-    {{2, 1, 2, 4}, {{2, 0.12f, 0.73f}, {2, 0.06f, 0.77f}, {0, 0.f, 0.f}, {1, 0.f, 0.91f}}},
-    {{2, 2, 2, 4}, {{1, 0.f, 1.38f}, {1, 0.f, 1.41f}, {1, 0.f, 1.73f}, {1, 0.f, 1.70f}}},
-    {{2, 1, 4, 4}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {1, 0.f, 1.56f}}},
-    {{4, 1, 4, 2}, {{2, 0.07f, 0.99f}, {1, 0.f, 0.99f}, {4, 0.22f, 1.05f}, {1, 0.f, 1.10f}}},
+    {{2, 1, 2, 4}, {{2, 0.12f, 0.73f}, {2, 0.06f, 0.77f}, {0, 0.f, 0.f}, {1, 0.42f, 0.87f}}},
+    {{2, 2, 2, 4}, {{1, 0.f, 1.38f}, {1, 0.f, 1.41f}, {1, 0.f, 1.73f}, {1, 0.22f, 1.77f}}},
+    {{2, 1, 4, 4}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {1, 0.47f, 1.43f}}},
+    {{4, 1, 4, 2}, {{2, 0.07f, 0.99f}, {1, 0.f, 0.99f}, {4, 0.22f, 1.05f}, {1, 0.21f, 1.15f}}},
     {{4, 2, 4, 2}, {{1, 0.f, 1.83f}, {1, 0.f, 1.71f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
     {{4, 2, 4, 1}, {{3, 0.54f, 0.68f}, {0, 0.f, 0.f}, {4, 0.45f, 0.76f}, {0, 0.f, 0.f}}},
-    {{4, 1, 8, 2}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {1, 0.f, 1.65f}}},
+    {{4, 1, 8, 2}, {{0, 0.f, 0.f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}, {3, 0.49f, 1.71f}}},
     {{4, 2, 8, 1}, {{2, 1.10f, 1.17f}, {4, 0.35f, 1.10f}, {0, 0.f, 0.f}, {0, 0.f, 0.f}}},
     {{4, 2, 8, 2}, {{1, 0.f, 3.54f}, {0, 0.f, 0.f}, {2, 0.05f, 3.51f}, {0, 0.f, 0.f}}},
-    {{8, 1, 8, 1}, {{0, 0.f, 0.f}, {1, 0.f, 1.35f}, {3, 0.43f, 1.57f}, {1, 0.f, 1.39f}}},
+    {{8, 1, 8, 1}, {{0, 0.f, 0.f}, {1, 0.f, 1.35f}, {3, 0.43f, 1.57f}, {3, 0.13f, 1.47f}}},
     {{8, 2, 8, 1}, {{1, 0.f, 3.07f}, {1, 0.f, 2.24f}, {1, 0.f, 3.43f}, {0, 0.f, 0.f}}},
 };
 
