@@ -399,23 +399,29 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
   return gemm_lds_bytes(fmt, q, static_cast<int>(k)) <= kLdsMax;
 }
 
-// The tiled GEMM (gemm_tile.h) takes every batch whose rows are long enough.  Measured on MI355X against gemm.hip's kernel
-// (graph replays, cold weights) over 10 shapes (127 x 4096 to 28672 x 4096) and 14 column counts from 4 to 2048 it is
-// faster at nearly all of them: Q4_0 28672 x 4096 at 16 columns 30.8 -> 20.1 us, 14336 x 4096 at 64 columns 35 -> 24, at
-// 512 columns 385 -> 105, Q8_0 14336 x 4096 at 16 columns 24.3 -> 14.1, TQ2_0 6912 x 2560 at 8 columns 6.3 -> 4.7, at 2048
-// columns 326 -> 61, Q4_K 4096 x 14336 at 1001 columns 561 -> 181.  gemm.hip's kernel keeps
-//   rows of at most 4 K steps, which are over before the tile's staging pays;
-//   up to 8 columns over at most a row a CU (Q4_0 127 x 4192 5.1 us against 5.3, TQ2_0 127 x 2816 3.8 against 4.1; Q8_0 is
-//     as fast on the tile) and, of the 4-bit formats' long rows, over one row tile a CU (Q4_0 4096 x 14336 at 4 columns
-//     12.7 against 13.6; 4096 x 4096 5.7 against 5.5);
-//   Q8_0 up to 16 columns just past one row tile a CU (4097 x 4192 at 8 columns 9.7 against 11.2; 6144 x 4096 11.9 against
-//     9.1);
-//   Q4_K's few columns, whose scale products the tile multiplies into the weights once per column group: up to 8 columns
-//     (4096 x 14336 13.3 us against 16.3, 28672 x 4096 at 5 columns 24.8 against 25.3); up to 16 over at most 2 row tiles a
-//     CU where rows are long or few (2560 x 6912 at 16 columns 9.2 against 9.8, 127 x 2816 5.1 against 6.1; 4096 x 4096 7.6
-//     against 7.0 goes to the tile); up to 32 where two column groups are just past a workgroup a CU (2560 x 6912 at 24
-//     columns 11.6 against 12.8); and 49-64 columns over about one row tile a CU, where komp_gemm_plan's answer of one group
-//     of 64 columns is part of the interface (the tile's two groups would take 4096 x 14336 in 31.5 us against 42).
+// The tiled GEMM (gemm_tile.h) takes every batch whose rows are longer than 4 K steps (before that they are over before its
+// staging pays), except where the batched kernel of gemm.hip is the faster one.  Measured on MI355X against that kernel (graph
+// replays over rotating weights; 25000 points: 64 to 128256 rows, 672 to 14336 values of K, 1 to 128 columns), the tile is
+// mostly 1.2-3 times as fast from 17 columns on (Q4_0 14336 x 4096 at 64 columns 35 -> 24 us, TQ2_0 6912 x 2560 at 2048 columns
+// 326 -> 61).  batched_keeps holds the rest, to within 0.2% of the faster kernel on average.  With few columns the batched
+// kernel's waves hold less: up to 16 columns a tile computes 16 in any case.  What decides (us, batched kernel / tile):
+//   rows: up to one 16-row tile a CU the batched kernel's workgroups fill the chip in one round.  Past it they need two, and
+//     the tile takes 32 rows a workgroup: Q4_0 4096 x 2560 at 4 columns 4.7 / 5.6, 6144 x 2560 6.8 / 6.5; Q8_0 4608 x 4096 10.2
+//     / 7.9, at 16 columns 14.8 / 9.2.  (At 4097-4100 rows, where the second round is a row or two, the tile is 3-15% slower.)
+//   K: the tile's 8 K groups compute their idle steps too.  Where the last round leaves more than 12% idle (`ragged`), the
+//     4-bit formats keep up to 12 columns (Q4_0 4096 x 2560, 20 steps in 24, at 12 columns 5.2 / 5.7; at 16 5.6 / 5.7), TQ2_0 8
+//     (2560 x 6912, 27 in 32, at 4 columns 5.4 / 6.3, at 9 6.1 / 6.3), Q8_0 4 (4096 x 1280 4.2 / 4.5; at 8 4.5 / 4.5); with no
+//     idle steps Q4_0 6-8 (4096 x 14336 at 4 columns 11.9 / 13.0, at 12 15.3 / 14.9), TQ2_0 2 (2560 x 8192 at 4 6.3 / 6.2).
+//   4-bit formats past one row tile a CU, long rows, where the batched kernel's rounds come out even: up to 2 tiles a CU (Q4_0
+//     6144 x 6912 at 4 columns 11.1 / 11.2) and 3-4 (14336 x 6912 at 8 columns 20.1 / 20.9; 10240 x 6912 at 4 17.8 / 16.9).
+//     IQ4_NL at 17-24 columns over 6-8 (28672 x 4096 at 17 columns 30.7 / 35.6; 24576 x 4096 at 24 7% the other way).
+//   Q4_K: the tile multiplies the scales into the weights once per column group, so its first columns cost the most, and a
+//     17th or 33rd column another group: 2048 x 6912 at 16 columns 8.9 / 9.9, 2560 x 6912 at 17 10.2 / 13.4, at 32 12.6 / 13.5,
+//     4096 x 6912 at 33 14.2 / 17.3, at 48 16.8 / 17.6; without idle K groups 4096 x 4096 at 16 7.3 / 7.0, at 24 8.9 / 8.9, at
+//     32 9.7 / 9.1; past one row tile a CU 6912 x 4096 at 8 8.3 / 9.2, at 16 10.6 / 9.3, 14336 x 4096 at 8 13.9 / 14.3, at 12
+//     15.6 / 14.5, 32768 x 4096 at 8 24.6 / 25.8, at 12 28.0 / 26.3.
+//   Q4_K at 49-64 columns over about one row tile a CU and rows of up to 16 blocks runs the batched kernel though the tile is
+//     faster (4096 x 4096 at 64 columns 15.3 / 11.8): komp_gemm_plan's answer there, one group of 64 columns, is tested.
 //
 // The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
@@ -451,21 +457,39 @@ constexpr TileCost kTileCosts[] = {
     {{8, 2, 8, 1}, {{1, 0.f, 3.07f}, {1, 0.f, 2.24f}, {1, 0.f, 3.43f}, {0, 0.f, 0.f}}},
 };
 
+// Whether gemm.hip's kernel keeps a call (the measurements are above).  units: what the K groups share out, K steps or
+// (Q4_K) blocks.
+bool batched_keeps(int fmt, int64_t m, int64_t n, int64_t nblk, int64_t units) {
+  const int64_t cus = device_cus();
+  const int64_t idle = (units + 7) / 8 * 8 - units;  // of 8 K groups' last round
+  const bool some = 100 * idle > 3 * units, ragged = 100 * idle > 12 * units;
+  switch (fmt) {
+    case FMT_Q4_0:
+    case FMT_IQ4_NL:
+      if (fmt == FMT_IQ4_NL && m > 16 && m <= 24 && n > 96 * cus && n <= 128 * cus && units > 8) return true;
+      if (n <= 16 * cus) return m <= (ragged ? 12 : fmt == FMT_IQ4_NL ? 3 : units > 60 ? 8 : 6);
+      return units > 40 && ((n <= 32 * cus && m <= 4) || (n > 48 * cus && n <= 64 * cus && m <= 8));
+    case FMT_Q8_0: return n <= 16 * cus && ragged && m <= 4;
+    case FMT_TQ2_0: return n <= 16 * cus && m <= (units <= 8 || !some ? 2 : ragged ? 8 : 5);
+    default:  // Q4_K
+      if (m > 48 && m <= 64 && n > 8 * cus && n <= 16 * cus && nblk <= 16) return true;
+      if (n <= 8 * cus) return m <= (some ? 16 : 12);
+      if (n <= 16 * cus && some) return m <= (n <= 10 * cus ? 32 : 40);
+      if (n <= 16 * cus)
+        return m <= 12 || (m <= 24 && (m > 16 || units > 32)) || (n > 10 * cus && units > 32 && m > 32 && m <= 40);
+      return m <= (n <= 32 * cus && ragged ? 16 : n <= 32 * cus ? 10 : n <= 64 * cus ? 9 : 8);
+  }
+}
+
 // False when the call stays on gemm.hip's kernel: by the rules above, or past the tile's 32-bit buffer offsets (128 rows
 // of SW bytes, 128 columns of K).
 bool gemm_tile_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, TilePlan* p) {
   const int64_t nblk = k / fmt_info(fmt).block;
   const int64_t steps = fmt == FMT_Q4_K ? 2 * nblk : fmt == FMT_TQ2_0 ? nblk : (nblk + 3) / 4;
   const int64_t cus = device_cus();
-  const bool blk32 = fmt_info(fmt).block == 32;
   if (steps <= 4 || n < 1) return false;
   if (128 * k > 0x7FFFFFF0 || 128 * sw > 0x7FFFFFF0) return false;
-  if (fmt == FMT_Q4_K && (m <= 8 || (m <= 16 && n <= 32 * cus && (nblk > 24 || n <= cus)) ||
-                          (m <= 32 && n > 8 * cus && n <= 12 * cus) ||
-                          (m > 48 && m <= 64 && n > 8 * cus && n <= 16 * cus)))
-    return false;
-  if (m <= 8 && ((fmt != FMT_Q8_0 && n <= cus) || (blk32 && fmt != FMT_Q8_0 && nblk > 256 && n <= 16 * cus))) return false;
-  if (m <= 16 && fmt == FMT_Q8_0 && n > 16 * cus && n <= 20 * cus) return false;
+  if (batched_keeps(fmt, m, n, nblk, fmt == FMT_Q4_K ? nblk : steps)) return false;
   const int row = fmt == FMT_TQ2_0 ? 1 : fmt == FMT_Q8_0 ? 2 : fmt == FMT_Q4_K ? 3 : 0;
   double best = -1;
   for (const TileCost& t : kTileCosts) {
