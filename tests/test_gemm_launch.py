@@ -1,8 +1,12 @@
 """Which matrix-core GEMM launch a call makes (the library's plan query; no GPU needed)."""
 
+import os
+import re
+
 import pytest
 
 from comp_amd import _abi, host
+from tests import test_gpu_gemm_tile as tile_tests
 
 FMTS = sorted(host.FMT_ID)
 
@@ -90,3 +94,35 @@ MEASURED = [
 @pytest.mark.parametrize("fmt,m,n,k,tiled", MEASURED)
 def test_the_faster_kernel_runs(fmt, m, n, k, tiled):
     assert launch(fmt, m, n, k)[0] == tiled
+
+
+CSRC = os.path.join(os.path.dirname(_abi.__file__), "csrc")
+
+
+def built(fmt):
+    """(row groups, row tiles, column tiles, K groups) of the tiled plans that the source builds for a format."""
+    flags = dict(q4=fmt in ("q4_0", "iq4_nl"), tq2=fmt == "tq2_0", q8=fmt == "q8_0", qk=fmt == "q4_k", true=True)
+    with open(os.path.join(CSRC, "gemm_tile.h")) as f:
+        lines = re.findall(r"^  KOMP_TILE_PLAN\(([^()]*)\)", f.read(), re.M)
+    plans = [line.split(",") for line in lines]
+    return {tuple(map(int, p[1:])) for p in plans if eval(p[0].replace("||", " or ").replace("!", " not "), {}, flags)}
+
+
+def reached(fmt):
+    """(tiled, K groups, row groups, row tiles, column tiles) of launches over a grid of shapes, on 256 CUs."""
+    blk = host.FORMATS[fmt]["block"]
+    cols = (1, 4, 8, 12, 14, 16, 17, 20, 24, 32, 33, 40, 48, 49, 64, 65, 96, 128, 130, 200, 333, 515, 1024, 1100, 2048)
+    rows = (64, 300, 700, 1500, 2560, 3584, 4096, 5200, 6912, 8400, 9216, 11000, 12330, 14336, 16500, 20000, 24576, 28700, 40000)
+    values = (672, 736, 1280, 1536, 2048, 2560, 4096, 6912, 8192, 14336)
+    return {launch(fmt, m, n, k)[:5] for m in cols for n in rows for k in values if k % blk == 0}
+
+
+@pytest.mark.parametrize("fmt", FMTS)
+def test_every_tiled_plan_is_built_reached_and_tested(fmt):
+    want = {(wk, rw, wn, cn) for rw, wn, cn, wk in built(fmt)}
+    assert {p[1:] for p in reached(fmt) if p[0]} == want
+    long = host.FORMATS[fmt]["block"] == 256
+    shapes = [(n, k256 if long else k32, m) for n, k32, k256, m in tile_tests.RAGGED]
+    shapes += [(n, 1536 if long else 736, m) for n, m in tile_tests.PLANS]
+    shapes += [(n, k, m) for f, n, k, m, *_ in (*tile_tests.MORE, *tile_tests.REST) if f == fmt]
+    assert {p[1:] for p in (launch(fmt, m, n, k)[:5] for n, k, m in shapes) if p[0]} == want

@@ -1,12 +1,12 @@
 """The tiled matrix-core GEMM (komp_*_gemm, rows of more than 4 K steps): S exact and Y within its bound against the oracle on
-ragged shapes (rows, columns and blocks that leave partial tiles, steps and K groups), and on shapes large enough for
-every plan, where the exact block dots are f64 matrix products of the oracle's decoded weights."""
+ragged shapes (rows, columns and blocks that leave partial tiles, steps and K groups; a few of few columns run the batched
+kernel), and on shapes large enough for every plan, where the exact block dots are f64 matrix products of the oracle's decoded weights."""
 
 import numpy as np
 import pytest
 import torch
 
-from comp_amd import host
+from comp_amd import _abi, host
 from oracle import oracle as O
 from tests.test_gpu_gemm import check, dev
 
@@ -31,7 +31,8 @@ def test_unaligned_scales_and_padded_rows(fmt):
     check(fmt, 45, k, 66, 21, ws_offset=8 if fmt == "q4_k" else 1, pad=48)
 
 
-# (n, m) at 1280 or 672 values of K: together they take every plan of gemm_tile_plan on a 256-CU device
+# (n, m) at 1536 or 736 values of K: with MORE and REST every plan of gemm_tile_plan on a 256-CU device, in every format
+# (tests/test_gemm_launch.py holds the lists to that)
 PLANS = [(64, 5), (4331, 5), (8400, 9), (1420, 33), (4331, 20), (8400, 20), (2340, 200), (5340, 49), (8400, 33), (670, 768),
          (8400, 66), (8400, 130), (11000, 130), (12330, 200), (11000, 260), (11000, 515)]
 
@@ -43,7 +44,7 @@ def test_every_plan(fmt, shape):
     check_large(fmt, n, 1536 if O.FORMATS[fmt]["block"] == 256 else 736, m, shape)
 
 
-# the plans of gemm_tile_plan that the shapes above do not take, on a 256-CU device
+# plans that the shapes above do not take, on a 256-CU device
 MORE = [("q4_0", 28700, 1056, 66), ("iq4_nl", 4099, 1056, 5), ("q4_0", 12330, 672, 17), ("q4_0", 16500, 672, 1100),
         ("tq2_0", 70, 2304, 9), ("tq2_0", 4099, 2304, 5), ("tq2_0", 28700, 1536, 260), ("tq2_0", 28700, 1536, 5),
         ("q8_0", 20000, 672, 768), ("q8_0", 12330, 672, 17), ("q4_k", 4099, 2304, 9), ("q4_k", 8211, 1792, 17)]
@@ -51,6 +52,21 @@ MORE = [("q4_0", 28700, 1056, 66), ("iq4_nl", 4099, 1056, 5), ("q4_0", 12330, 67
 
 @pytest.mark.parametrize("fmt,n,k,m", MORE)
 def test_more_plans(fmt, n, k, m):
+    check_large(fmt, n, k, m, n + m)
+
+
+# (format, n, k, m, the workgroup's K groups, row groups, row tiles and column tiles on a 256-CU device)
+REST = [("q4_0", 4331, 1280, 5, (4, 1, 2, 1)), ("q4_0", 6912, 1280, 17, (4, 2, 1, 2)), ("iq4_nl", 28700, 1280, 130, (1, 4, 2, 4)),
+        ("iq4_nl", 16500, 672, 1100, (1, 4, 2, 8)), ("iq4_nl", 6912, 1280, 17, (4, 2, 1, 2)),
+        ("iq4_nl", 12330, 672, 17, (4, 2, 2, 2)), ("q4_k", 8400, 1280, 12, (4, 1, 2, 1))]  # fmt: skip
+
+
+@pytest.mark.parametrize("fmt,n,k,m,plan", REST)
+def test_remaining_plans(fmt, n, k, m, plan):
+    f = host.FORMATS[fmt]
+    launch = _abi.gemm_launch(host.FMT_ID[fmt], m, n, k, k // f["block"] * f["qbytes"])
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert launch[:5] == (True, *plan)
     check_large(fmt, n, k, m, n + m)
 
 

@@ -65,3 +65,42 @@ def test_accepted_forms_on_another_stream(fmt):
     assert torch.equal(xq, t["xq"]) and torch.equal(xd, t["xd"])
     for v in (y, y2):
         assert outputs_ok(fmt, v.cpu().numpy(), ws, rd, rs, r)
+
+
+@pytest.mark.parametrize("entry", ["quantize", "gemv", "gemm", "gemv_f32", "split"])
+def test_captured_launches_are_on_the_capturing_stream(entry):
+    """Each entry captured on a stream that is not the default one: the replays compute from inputs written after the
+    capture, so the launch is in the graph and not on some other stream."""
+    t, _, n, k = setup()
+    x2 = torch.randn_like(t["x"])
+    blocks = torch.randint(0, 256, (n * (k // 32) * 18,), dtype=torch.uint8, device="cuda")
+    xq, xd = torch.empty_like(t["xq"]), torch.empty_like(t["xd"])
+    y = torch.empty((t["x"].shape[0], n), device="cuda")
+    wq, ws = torch.empty_like(t["wq"]), torch.empty_like(t["ws"])
+    call, outs = {
+        "quantize": (lambda: host.quantize_into("q4_0", t["x"], xq, xd), (xq, xd)),
+        "gemv": (lambda: host.gemv_into("q4_0", t["wq"], t["ws"], t["xq"], t["xd"], y, n, k), (y,)),
+        "gemm": (lambda: host.gemm_into("q4_0", t["wq"], t["ws"], t["xq"], t["xd"], y, n, k), (y,)),
+        "gemv_f32": (lambda: host.gemv_f32_into("q4_0", t["wq"], t["ws"], t["x"], y, n, k), (y,)),
+        "split": (lambda: host.split_into("q4_0", blocks, wq, ws, n, k), (wq, ws)),
+    }[entry]
+    call()  # loads the kernel
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        call()
+    torch.cuda.synchronize()
+    for i in range(3):
+        t["x"].copy_(x2 * (i + 1))
+        q2, d2 = host.quantize("q4_0", t["x"])
+        t["xq"].copy_(q2)
+        t["xd"].copy_(d2)
+        blocks.add_(1)
+        call()
+        want = [o.clone() for o in outs]
+        for o in outs:
+            o.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(outs, want)) and any(bool(o.any()) for o in outs)

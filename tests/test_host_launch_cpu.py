@@ -1,6 +1,7 @@
 """How comp_amd.host reaches the library, without a GPU: what importing it needs of torch, which
-library its calls go to, and what they hand over and return."""
+library its calls go to, what they hand over and return, and on which device and stream they launch."""
 
+import contextlib
 import os
 import subprocess
 import sys
@@ -59,3 +60,44 @@ def test_outputs_are_plain_tensors_whatever_the_inputs_type(monkeypatch):
     assert [(tuple(t.shape), t.dtype) for t in q] == [
         ((2, 1024), torch.int8), ((2, 32), torch.float32),
         ((2, 1024), torch.int8), ((2, 4), torch.float32), ((2, 64), torch.int16)]  # fmt: skip
+
+
+class OnDeviceOne(DeviceLike):
+    def get_device(self):
+        return 1
+
+
+def test_launches_pass_the_tensors_devices_current_stream(monkeypatch):
+    """The stream is the last argument, and the device is switched for the call alone, if it is another one."""
+    log, current = [], [0]
+
+    @contextlib.contextmanager
+    def switched(dev):
+        before, current[0] = current[0], dev
+        log.append(("switch", dev))
+        yield
+        current[0] = before
+
+    def entry(name):
+        return lambda *a: log.append((name, current[0], a[-1])) or 0
+
+    monkeypatch.setattr(_abi, "entry", entry)
+    monkeypatch.setattr(host, "_raw_stream", lambda dev: 1000 + dev)
+    monkeypatch.setattr(host, "_current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "device", switched)
+    monkeypatch.setattr(host, "_weights_fit", lambda *a: True)
+    like = lambda t: t.as_subclass(OnDeviceOne)  # noqa: E731
+    w, ws = like(torch.zeros((8, 512), dtype=torch.uint8)), like(torch.zeros((8, 32), dtype=torch.int16))
+    x, xq, xd = like(torch.zeros((2, 1024))), like(torch.zeros((2, 1024), dtype=torch.int8)), like(torch.zeros((2, 32)))
+    monkeypatch.setattr(host, "_plain", lambda t: t)  # the device stays the fake one
+    for call, name in (
+        (lambda: host.quantize("q4_0", x), "komp_quant_q8_0"),
+        (lambda: host.gemv("q4_0", w, ws, xq, xd, 8, 1024), "komp_q4_0_gemv"),
+        (lambda: host.gemm("q4_0", w, ws, xq, xd, 8, 1024), "komp_q4_0_gemm"),
+        (lambda: host.gemv_f32("q4_0", w, ws, x, 8, 1024), "komp_q4_0_gemv_f32"),
+    ):
+        for at in (0, 1):
+            current[0] = at
+            log.clear()
+            call()
+            assert log == ([("switch", 1)] if at == 0 else []) + [(name, 1, 1001)] and current[0] == at
