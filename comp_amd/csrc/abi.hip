@@ -320,8 +320,8 @@ GemvPlan knob_plan(int fmt, int block_n, int nb, int num_warps) {
 }
 
 // ---- matrix-core GEMM ----------------------------------------------------------------------------------------------
-// From kGemmMinM activation columns on, block_n == 0 in dp4a mode (unfused) runs the matrix-core GEMM, which reads the
-// weights once per 64 columns, instead of the GEMV in column chunks of 3 (which reads them once for up to 3 columns,
+// From kGemmMinM activation columns on, block_n == 0 in dp4a mode (unfused) runs a matrix-core GEMM, which reads the
+// weights once per 16-128 columns, instead of the GEMV in column chunks of 3 (which reads them once for up to 3 columns,
 // in one launch).  At 4 columns the GEMM is 1.2-1.8x faster at Llama-3-8B and BitNet-2B shapes; at 3 the lean GEMVs
 // are as fast or faster (TQ2_0 6912 x 2560: 5.6 against 5.8 us, 2560 x 6912: 5.7 against 5.2, 32768 x 8192: 22.5
 // against 23.9; Q4_0 4096 x 14336: 9.9 against 13.9).
@@ -331,9 +331,12 @@ constexpr int64_t kGemmMaxCols = 16 * 65535;  // columns per GEMM launch: at mos
 // The GEMM's plan for m columns (one launch) and n rows.  Columns go in groups of at most 64 (4 tiles of 16), split
 // evenly.  The waves of a workgroup split K (wk) and rows (wr) by how many 16-row tiles each CU gets (r, counting
 // column groups): with about one per CU every wave of a CU must share the tile's K, so K is split 8 ways; with a few
-// per CU, 2-4 ways; with many, each wave owns its rows and no partial sums meet.  Measured on MI355X at Llama-3-8B
-// (4096x4096, 14336x4096, 4096x14336, 128256x4096) and BitNet-2B shapes, 1..64 columns.  False when the shape is past
-// the kernel's 32-bit buffer offsets (64 * K and 32 * SW below 2^31) or its scale slab does not fit in LDS.
+// per CU, 2-4 ways; with many, each wave owns its rows and no partial sums meet.  The lines were drawn when this kernel ran
+// every batch, measured on MI355X at Llama-3-8B (4096x4096, 14336x4096, 4096x14336, 128256x4096) and BitNet-2B shapes,
+// 1..64 columns.  Of these the tiled kernel has since taken most (batched_keeps): past 16 columns only rows of up to 4 K
+// steps, a few of Q4_K's and IQ4_NL's shapes and no plan of 8 K groups by 4 column tiles (but Q4_K's) are left here.  False
+// when the shape is past the kernel's 32-bit buffer offsets (64 * K and 32 * SW below 2^31) or its scale slab does not fit in
+// LDS; the tiled kernel, which has no slab, keeps to the same limits.
 bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p) {
   if (64 * k > INT32_MAX || 32 * sw > INT32_MAX) return false;
   if (fmt == FMT_Q4_K) {
@@ -361,7 +364,7 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
   double r = static_cast<double>(tiles) * groups / device_cus();
   // Few row tiles a CU: fewer column tiles a workgroup, in more column groups (each reads its rows' weights again,
   // mostly from L2).  4 column tiles and at most 2 row tiles a CU: halve until each CU has more than 2; at 64 columns
-  // Q4_0 4096 x 4096 16.3 -> 15.0 us, 4096 x 14336 46.0 -> 40.2, TQ2_0 2560 x 6912 18.6 -> 14.7 (one column tile a
+  // (of rows that the tiled kernel now runs) Q4_0 4096 x 4096 16.3 -> 15.0 us, 4096 x 14336 46.0 -> 40.2, TQ2_0 2560 x 6912 18.6 -> 14.7 (one column tile a
   // workgroup), TQ2_0 6912 x 2560 14.7 -> 12.0 (two).  3 column tiles with idle CUs: one column tile a workgroup
   // (TQ2_0 2560 x 6912 at 48 columns 14.5 -> 11.9 us; at 4096 rows, one tile a CU, splitting measured slower).
   const auto regroup = [&](int to) {

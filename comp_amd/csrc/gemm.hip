@@ -3,8 +3,8 @@
 //   Y[m][n] = sum_b d_w(n, b) * d_x(m, b) * s(m, n, b),  s = the exact int32 dot of weight block b of row n with
 //   activation block b of column m,
 // and the same optional S [M][N][K/block] of exact block dots.  The GEMVs stream the weights once per 1..3 columns;
-// this kernel streams them once per 64 columns, so a batch of decode tokens reads each weight byte once.  Larger batches
-// and prompts run the tiled kernel of gemm_tile.h (gemm_tile_plan in abi.hip says from where).
+// this kernel streams them once per 64 columns.  It runs rows of up to 4 K steps and the small batches at which it is the
+// faster one (batched_keeps in abi.hip); the others, from 4 columns to prompts, run the tiled kernel of gemm_tile.h.
 //
 // Tiles.  A workgroup (W waves) owns 16*WN weight rows x 16*CN activation columns and all of K.  Its waves split K:
 // a K step is 64 contiguous bytes of each weight row (4 Q4_0 blocks or 1 TQ2_0 block) and wave w takes steps
@@ -12,7 +12,7 @@
 // g = lane / 16) loads bytes 16g..16g+15 of a step for row r, so one load instruction reads 64 bytes of each of 16
 // rows.  Each wave keeps D steps of activation loads and DW >= D steps of weight loads in flight (register rings;
 // the step loop has no branch, so each step waits for its own loads only).  Loads go through buffer descriptors whose
-// range ends at the tile's last valid row / column, with the whole offset of a load in its per-lane offset (no scalar
+// range ends with the tile's last valid row's blocks / column, with the whole offset of a load in its per-lane offset (no scalar
 // offset): a load past the range (a block past K in the tile's last row, every load of a step past the wave's last)
 // returns zeros without touching memory.
 //
@@ -609,10 +609,8 @@ hipError_t launch_fmt(const GemmCall& c, const GemmPlan& p, hipStream_t stream) 
   KOMP_GEMM_PLAN(8, 1, 1, 1, 2)
   KOMP_GEMM_PLAN(8, 1, 1, 2, 2)
   KOMP_GEMM_PLAN(8, 1, 1, 3, 2)
-  KOMP_GEMM_PLAN(8, 1, 1, 4, 2)
   KOMP_GEMM_PLAN(4, 2, 1, 2, 2)
   KOMP_GEMM_PLAN(4, 2, 1, 3, 2)
-  KOMP_GEMM_PLAN(4, 2, 1, 4, 2)
   KOMP_GEMM_PLAN(4, 2, 2, 1, 4)
   KOMP_GEMM_PLAN(2, 4, 1, 2, 2)
   KOMP_GEMM_PLAN(2, 4, 1, 3, 2)

@@ -298,7 +298,7 @@ def gemm(fmt, wq, ws, xq, xd, n, k, store_s=False):
     """-> (Y f32 [M][N], S int32 [M][N][blocks] or None) on the matrix cores, for any number M of columns.
 
     The result definition of gemv (exact int32 block dots, then d_w * d_x scaling, src/komp/kernels.py:48-142); the
-    weights are read once per 64 columns.  gemv(..., block_n=None, mode=2) runs this kernel from GEMM_MIN_M columns
+    weights are read once per 16 to 128 columns.  gemv(..., block_n=None, mode=2) runs this kernel from GEMM_MIN_M columns
     on."""
     m, nblk = _check_gemv(fmt, wq, ws, xq, xd, n, k)
     y = _plain(xd).new_empty((m, n))

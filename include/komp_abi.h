@@ -175,15 +175,14 @@ int komp_gemv_auto_config(int fmt, int fused, int mode, int64_t M, int64_t N, in
                           int* num_warps, int* lanes_per_row, int* passes);
 
 /* Y [M][N] (and S when not NULL) as komp_q4_0_gemv / komp_tq2_0_gemv compute them, for any M, on the matrix cores
- * (v_mfma_i32_16x16x32_i8 / v_mfma_i32_16x16x64_i8): each workgroup reads its weight rows once for up to 64
- * activation columns, where the GEMVs read them once per 3.  S is bit-identical to the GEMVs'; Y agrees to f32
+ * (v_mfma_i32_16x16x32_i8 / v_mfma_i32_16x16x64_i8 / v_mfma_f32_16x16x32_f16): each workgroup reads its weight rows once
+ * for 16 to 128 activation columns, where the GEMVs read them once per 3.  S is bit-identical to the GEMVs'; Y agrees to f32
  * rounding (the f32 sums run in another order).  Arguments and alignment as komp_q4_0_gemv / komp_tq2_0_gemv without
  * the knobs; also 64*K and 32*SW must be below 2^31 and the 16 or 32 rows of WS a workgroup stages must fit in LDS
  * (komp_gemm_plan says whether a shape qualifies).  komp_q4_0_gemv / komp_tq2_0_gemv with block_n == 0 and
  * KOMP_MODE_DP4A run this kernel for M >= 4 when the shape qualifies.
- * Rows of more than 4 K steps (512 values; TQ2_0 1024) run a tiled kernel (Q4_K: from 9-65 columns on, by the rows) that
- * stages the activations in LDS and reads the weights once per 16-128 columns, with the same S and the same Y to f32
- * rounding.
+ * Of two kernels, a batched one and a tiled one that stages the activations in LDS, the library runs the faster for the
+ * shape (komp_gemm_launch says which), with the same S and the same Y to f32 rounding.
  * No reference counterpart: the reference launches its GEMV once per column (grid (cdiv(N, BLOCK_N), M),
  * src/komp/kernels.py:50); this serves batched decode, where M columns share every weight byte. */
 int komp_q4_0_gemm(const uint8_t* WQ, const int16_t* WS, const int8_t* XQ, const float* XD, float* Y, int32_t* S,

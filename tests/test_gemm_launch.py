@@ -126,3 +126,12 @@ def test_every_tiled_plan_is_built_reached_and_tested(fmt):
     shapes += [(n, 1536 if long else 736, m) for n, m in tile_tests.PLANS]
     shapes += [(n, k, m) for f, n, k, m, *_ in (*tile_tests.MORE, *tile_tests.REST) if f == fmt]
     assert {p[1:] for p in (launch(fmt, m, n, k)[:5] for n, k, m in shapes) if p[0]} == want
+
+
+@pytest.mark.parametrize("fmt", [f for f in FMTS if f != "q4_k"])
+def test_batched_plans_that_are_not_built_are_not_asked_for(fmt):
+    """Eight or four K groups by four column tiles: only rows that the tiled kernel runs would take them (Q4_K aside)."""
+    blk = host.FORMATS[fmt]["block"]
+    got = {launch(fmt, m, n, nb * blk) for m in (1, 9, 17, 20, 24, 40, 49, 64, 100, 128, 256) for n in range(1, 40000, 499)
+           for nb in (1, 2, 3, 4, 6, 8, 12, 16, 17, 100, 700, 2000)}  # fmt: skip
+    assert not {p[1:5] for p in got if p and not p[0]} & {(8, 1, 1, 4), (4, 2, 1, 4)}
