@@ -403,28 +403,31 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 }
 
 // The tiled GEMM (gemm_tile.h) takes every batch whose rows are longer than 4 K steps (before that they are over before its
-// staging pays), except where the batched kernel of gemm.hip is the faster one.  Measured on MI355X against that kernel (graph
-// replays over rotating weights; 25000 points: 64 to 128256 rows, 672 to 14336 values of K, 1 to 128 columns), the tile is
-// mostly 1.2-3 times as fast from 17 columns on (Q4_0 14336 x 4096 at 64 columns 35 -> 24 us, TQ2_0 6912 x 2560 at 2048 columns
-// 326 -> 61).  batched_keeps holds the rest, to within 0.2% of the faster kernel on average.  With few columns the batched
-// kernel's waves hold less: up to 16 columns a tile computes 16 in any case.  What decides (us, batched kernel / tile):
-//   rows: up to one 16-row tile a CU the batched kernel's workgroups fill the chip in one round.  Past it they need two, and
-//     the tile takes 32 rows a workgroup: Q4_0 4096 x 2560 at 4 columns 4.7 / 5.6, 6144 x 2560 6.8 / 6.5; Q8_0 4608 x 4096 10.2
-//     / 7.9, at 16 columns 14.8 / 9.2.  (At 4097-4100 rows, where the second round is a row or two, the tile is 3-15% slower.)
-//   K: the tile's 8 K groups compute their idle steps too.  Where the last round leaves more than 12% idle (`ragged`), the
-//     4-bit formats keep up to 12 columns (Q4_0 4096 x 2560, 20 steps in 24, at 12 columns 5.2 / 5.7; at 16 5.6 / 5.7), TQ2_0 8
-//     (2560 x 6912, 27 in 32, at 4 columns 5.4 / 6.3, at 9 6.1 / 6.3), Q8_0 4 (4096 x 1280 4.2 / 4.5; at 8 4.5 / 4.5); with no
-//     idle steps Q4_0 6-8 (4096 x 14336 at 4 columns 11.9 / 13.0, at 12 15.3 / 14.9), TQ2_0 2 (2560 x 8192 at 4 6.3 / 6.2).
-//   4-bit formats past one row tile a CU, long rows, where the batched kernel's rounds come out even: up to 2 tiles a CU (Q4_0
-//     6144 x 6912 at 4 columns 11.1 / 11.2) and 3-4 (14336 x 6912 at 8 columns 20.1 / 20.9; 10240 x 6912 at 4 17.8 / 16.9).
-//     IQ4_NL at 17-24 columns over 6-8 (28672 x 4096 at 17 columns 30.7 / 35.6; 24576 x 4096 at 24 7% the other way).
+// staging pays), except where the batched kernel of gemm.hip is the faster one.  Measured on MI355X against that kernel as a
+// decode step runs it (quantizer and GEMM, each layer with its own weights, inputs and q8 planes, graph replays), over 12600
+// points (64 to 128256 rows, 672 to 14336 values of K, 4 to 64 columns), with weights out of the caches (as those of a model
+// larger than them are at every token) and with weights that the replay before left there.  The two differ: the batched
+// kernel's weight loads are non-temporal, the tile's are not, so weights at rest make the tile 5-15% faster at few columns
+// where cold ones leave the kernels even.  batched_keeps holds the calls that lose nothing that way: those faster on the
+// batched kernel cold and no more than 3% slower warm.  What decides (tile's time over the batched kernel's, a quantizer and a
+// GEMM together, cold / warm):
+//   rows: up to one 16-row tile a CU the batched kernel's workgroups fill the chip in one round; past it they need two, and
+//     the tile takes 32 rows a workgroup: Q8_0 at 4 columns 0.93-0.97 / 0.86-0.93 up to 4096 rows, 0.84 / 0.80 at 4300-8192
+//     (0.67-0.82 at 16 columns), so Q8_0 has no case left but 4097-4100 rows, where the second round is a row or two (1.05-1.1).
+//   K: the tile's 8 K groups compute their idle steps too.  Where more than 12% of the last round is idle (`ragged`): Q4_0 and
+//     IQ4_NL with 20 steps at 4 columns 1.11 / 1.01, at 6 1.09 / 0.99, at 8 1.07 / 0.97, with 10-12 at 4 1.05 / 0.96; TQ2_0 (10-20) at 4 1.07 / 1.05, at 9 1.03 /
+//     1.01, at 12 1.00 / 0.98; 27 steps at 4 1.09 / 1.03, at 8 1.01 / 0.96.  With 3-12% idle TQ2_0 at 4 1.05 / 1.01, at 8 0.98 /
+//     0.93; with none 1.00 / 0.97.  Q4_0 with none, long rows: at 4 1.03 / 0.92, at 8 0.99 / 0.87.
+//   4-bit formats, long rows over 3-4 row tiles a CU, where the batched kernel's rounds come out even: Q4_0 at 4 1.07 / 1.08, at
+//     8 1.04 / 1.04, at 12 1.00; over 6-8 a 17th column, which costs the tile another column tile: Q4_0 at 17 1.05-1.11, at 24
+//     0.95-1.00, IQ4_NL at 17 1.11-1.25, at 24 1.04-1.13, at 32 0.97-1.02.
 //   Q4_K: the tile multiplies the scales into the weights once per column group, so its first columns cost the most, and a
-//     17th or 33rd column another group: 2048 x 6912 at 16 columns 8.9 / 9.9, 2560 x 6912 at 17 10.2 / 13.4, at 32 12.6 / 13.5,
-//     4096 x 6912 at 33 14.2 / 17.3, at 48 16.8 / 17.6; without idle K groups 4096 x 4096 at 16 7.3 / 7.0, at 24 8.9 / 8.9, at
-//     32 9.7 / 9.1; past one row tile a CU 6912 x 4096 at 8 8.3 / 9.2, at 16 10.6 / 9.3, 14336 x 4096 at 8 13.9 / 14.3, at 12
-//     15.6 / 14.5, 32768 x 4096 at 8 24.6 / 25.8, at 12 28.0 / 26.3.
+//     17th or 33rd column another group.  Up to half a row tile a CU at 12 columns 1.00-1.14 / 1.00-1.11, at 16 0.95-0.98 without
+//     and 1.03-1.09 with idle K groups; up to one at 17 1.05-1.25 / 1.03-1.22, at 33 (10 CUs' rows and more) 1.05-1.21, at 48
+//     0.95-1.04; up to two at 9 1.04-1.16, at 12 0.95 without and 1.07-1.09 with idle K groups; up to four at 9 1.01-1.12, at 14
+//     0.90-1.01; over 4-6 0.83-0.96 at 8 but for rows of 5-6 blocks (1.03 at 4); over 6-8 at 8 1.01-1.24, at 12 0.93-1.04.
 //   Q4_K at 49-64 columns over about one row tile a CU and rows of up to 16 blocks runs the batched kernel though the tile is
-//     faster (4096 x 4096 at 64 columns 15.3 / 11.8): komp_gemm_plan's answer there, one group of 64 columns, is tested.
+//     faster (4096 x 4096 at 64 columns 15.3 us against 11.8): komp_gemm_plan's answer there, one group of 64 columns, is tested.
 //
 // The plan is the one with the least estimated time.  A K step of one workgroup costs a CU `b` us of issue and, once per
 // round of co-resident workgroups (`slots` a CU, by LDS and registers), `a` us of latency that the round shares; every
@@ -469,18 +472,20 @@ bool batched_keeps(int fmt, int64_t m, int64_t n, int64_t nblk, int64_t units) {
   switch (fmt) {
     case FMT_Q4_0:
     case FMT_IQ4_NL:
-      if (fmt == FMT_IQ4_NL && m > 16 && m <= 24 && n > 96 * cus && n <= 128 * cus && units > 8) return true;
-      if (n <= 16 * cus) return m <= (ragged ? 12 : fmt == FMT_IQ4_NL ? 3 : units > 60 ? 8 : 6);
-      return units > 40 && ((n <= 32 * cus && m <= 4) || (n > 48 * cus && n <= 64 * cus && m <= 8));
-    case FMT_Q8_0: return n <= 16 * cus && ragged && m <= 4;
-    case FMT_TQ2_0: return n <= 16 * cus && m <= (units <= 8 || !some ? 2 : ragged ? 8 : 5);
+      if (n <= 16 * cus)
+        return (ragged && units > 8 && m <= (n <= cus ? 8 : units > 16 ? 6 : 0)) || (fmt == FMT_Q4_0 && units > 60 && m <= 6);
+      if (n > 48 * cus && n <= 64 * cus) return units > 40 && m <= 8;
+      return n > 96 * cus && n <= 128 * cus && m > 16 && (fmt == FMT_Q4_0 ? m <= 20 && units > 24 : m <= 24 && units > 8);
+    case FMT_Q8_0: return false;
+    case FMT_TQ2_0: return n <= 16 * cus && units > 8 && m <= (ragged ? (units <= 24 ? 9 : 6) : some ? 5 : 2);
     default:  // Q4_K
       if (m > 48 && m <= 64 && n > 8 * cus && n <= 16 * cus && nblk <= 16) return true;
       if (n <= 8 * cus) return m <= (some ? 16 : 12);
       if (n <= 16 * cus && some) return m <= (n <= 10 * cus ? 32 : 40);
       if (n <= 16 * cus)
         return m <= 12 || (m <= 24 && (m > 16 || units > 32)) || (n > 10 * cus && units > 32 && m > 32 && m <= 40);
-      return m <= (n <= 32 * cus && ragged ? 16 : n <= 32 * cus ? 10 : n <= 64 * cus ? 9 : 8);
+      if (n <= 64 * cus) return m <= (n > 32 * cus ? 9 : ragged ? 12 : 10);
+      return n > 96 * cus ? m <= 8 : units <= 6 && m <= 6;
   }
 }
 
