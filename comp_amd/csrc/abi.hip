@@ -415,9 +415,10 @@ bool gemm_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t sw, GemmPlan* p
 //     the tile takes 32 rows a workgroup: Q8_0 at 4 columns 0.93-0.97 / 0.86-0.93 up to 4096 rows, 0.84 / 0.80 at 4300-8192
 //     (0.67-0.82 at 16 columns), so Q8_0 has no case left but 4097-4100 rows, where the second round is a row or two (1.05-1.1).
 //   K: the tile's 8 K groups compute their idle steps too.  Where more than 12% of the last round is idle (`ragged`): Q4_0 and
-//     IQ4_NL with 20 steps at 4 columns 1.11 / 1.01, at 6 1.09 / 0.99, at 8 1.07 / 0.97, with 10-12 at 4 1.05 / 0.96; TQ2_0 (10-20) at 4 1.07 / 1.05, at 9 1.03 /
-//     1.01, at 12 1.00 / 0.98; 27 steps at 4 1.09 / 1.03, at 8 1.01 / 0.96.  With 3-12% idle TQ2_0 at 4 1.05 / 1.01, at 8 0.98 /
-//     0.93; with none 1.00 / 0.97.  Q4_0 with none, long rows: at 4 1.03 / 0.92, at 8 0.99 / 0.87.
+//     IQ4_NL with 20 steps at 4 columns 1.11 / 1.01, at 6 1.09 / 0.99, at 8 1.07 / 0.97, with 10-12 at 4 1.05 / 0.96; TQ2_0 with
+//     10-20 at 4 1.07 / 1.05, at 9 1.03 / 1.01, at 12 1.00 / 0.98, with 27 at 4 1.09 / 1.03, at 8 1.01 / 0.96.  With 3-12% idle
+//     TQ2_0 at 4 1.05 / 1.01, at 8 0.98 / 0.93; with none 1.00 / 0.97.  Q4_0 with none, long rows: at 4 1.03 / 0.92, at 8 0.99 /
+//     0.87.
 //   4-bit formats, long rows over 3-4 row tiles a CU, where the batched kernel's rounds come out even: Q4_0 at 4 1.07 / 1.08, at
 //     8 1.04 / 1.04, at 12 1.00; over 6-8 a 17th column, which costs the tile another column tile: Q4_0 at 17 1.05-1.11, at 24
 //     0.95-1.00, IQ4_NL at 17 1.11-1.25, at 24 1.04-1.13, at 32 0.97-1.02.

@@ -609,6 +609,9 @@ hipError_t launch_fmt(const GemmCall& c, const GemmPlan& p, hipStream_t stream) 
   KOMP_GEMM_PLAN(8, 1, 1, 1, 2)
   KOMP_GEMM_PLAN(8, 1, 1, 2, 2)
   KOMP_GEMM_PLAN(8, 1, 1, 3, 2)
+  if constexpr (FMT == FMT_Q4_0) {  // no call takes it any more: the instruction-mix report lists its loop
+    KOMP_GEMM_PLAN(8, 1, 1, 4, 2)
+  }
   KOMP_GEMM_PLAN(4, 2, 1, 2, 2)
   KOMP_GEMM_PLAN(4, 2, 1, 3, 2)
   KOMP_GEMM_PLAN(4, 2, 2, 1, 4)

@@ -139,7 +139,8 @@ def test_every_tiled_plan_is_built_reached_and_tested(fmt):
 
 @pytest.mark.parametrize("fmt", [f for f in FMTS if f != "q4_k"])
 def test_batched_plans_that_are_not_built_are_not_asked_for(fmt):
-    """Eight or four K groups by four column tiles: only rows that the tiled kernel runs would take them (Q4_K aside)."""
+    """Eight or four K groups by four column tiles: only rows that the tiled kernel runs would take them (Q4_K aside; the
+    first is built for Q4_0 alone, for the instruction-mix report)."""
     blk = host.FORMATS[fmt]["block"]
     got = {launch(fmt, m, n, nb * blk) for m in (1, 9, 17, 20, 24, 40, 49, 64, 100, 128, 256) for n in range(1, 40000, 499)
            for nb in (1, 2, 3, 4, 6, 8, 12, 16, 17, 100, 700, 2000)}  # fmt: skip
