@@ -117,14 +117,9 @@ def check(status, what):
     raise KompError(msg)
 
 
-def entry(name):
-    """An ABI function of the loaded library (which keeps it as an attribute after the first look)."""
-    return getattr(_lib or lib(), name)
-
-
 def call(name, *args):
     """Call an ABI function and raise on a nonzero status."""
-    check(entry(name)(*args), name)
+    check(getattr(_lib or lib(), name)(*args), name)
 
 
 def auto_plan(fmt_id, m, n, k, fused=False, mode=2):

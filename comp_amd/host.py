@@ -178,19 +178,15 @@ _Tensor, _U8, _I16, _I8, _F32 = torch.Tensor, torch.uint8, torch.int16, torch.in
 
 def _launch(name, t, *args):
     """Call a launching ABI entry on t's device, with that device's current stream as its last argument."""
+    fn = getattr(_abi._lib or _abi.lib(), name)
     dev = t.get_device()
     if dev == _current_device():
-        st = _abi.entry(name)(*args, _raw_stream(dev))
+        st = fn(*args, _raw_stream(dev))
     else:
         with torch.cuda.device(dev):
-            st = _abi.entry(name)(*args, _raw_stream(dev))
+            st = fn(*args, _raw_stream(dev))
     if st:
         _abi.check(st, name)
-
-
-def _plain(t):
-    """t as a torch.Tensor: what new_empty makes from a subclass is of that subclass."""
-    return t if type(t) is _Tensor else t.as_subclass(_Tensor)
 
 
 def _plane(t, dtype, shape, dev):
@@ -224,7 +220,9 @@ def quantize(fmt, x, bb=4, bsums=False):
     act = FORMATS[fmt]["act"]
     if not (isinstance(x, _Tensor) and x.is_cuda and x.dtype is _F32 and x.dim() == 2):
         _need(x, "x", torch.float32, 2)
-    x = _plain(x.contiguous())
+    x = x.contiguous()
+    if type(x) is not _Tensor:  # new_empty makes tensors of the input's type
+        x = x.as_subclass(_Tensor)
     m, k = x.shape
     blk = 32 if act == "q8_0" else 256
     if k % blk:
@@ -283,7 +281,7 @@ def gemv(fmt, wq, ws, xq, xd, n, k, block_n=32, nb=4, mode=0, num_warps=4, store
 
     src/komp/host.py:76-85.  block_n=None lets the library choose block_n, nb and num_warps for the shape."""
     m, nblk = _check_gemv(fmt, wq, ws, xq, xd, n, k)
-    y = _plain(xd).new_empty((m, n))
+    y = (xd if type(xd) is _Tensor else xd.as_subclass(_Tensor)).new_empty((m, n))
     s = torch.zeros(_s_shape(fmt, m, n, nblk), dtype=torch.int32, device=xq.device) if store_s else None
     _launch_gemv(fmt, wq, ws, xq, xd, y, s, n, k, block_n, nb, mode, num_warps)
     return y, s
@@ -301,7 +299,7 @@ def gemm(fmt, wq, ws, xq, xd, n, k, store_s=False):
     weights are read once per 16 to 128 columns.  gemv(..., block_n=None, mode=2) runs this kernel from GEMM_MIN_M columns
     on."""
     m, nblk = _check_gemv(fmt, wq, ws, xq, xd, n, k)
-    y = _plain(xd).new_empty((m, n))
+    y = (xd if type(xd) is _Tensor else xd.as_subclass(_Tensor)).new_empty((m, n))
     s = torch.zeros(_s_shape(fmt, m, n, nblk), dtype=torch.int32, device=xq.device) if store_s else None
     _launch_gemm(fmt, wq, ws, xq, xd, y, s, n, k)
     return y, s
@@ -463,7 +461,9 @@ def gemv_f32(fmt, wq, ws, x, n, k, block_n=None, nb=4, mode=2, num_warps=4, stor
     planes (and the q8_K bsums).  No reference counterpart (the reference launches the two kernels separately)."""
     if not (isinstance(x, _Tensor) and x.is_cuda and x.dtype is _F32 and x.dim() == 2):
         _need(x, "x", torch.float32, 2)
-    x = _plain(x.contiguous())
+    x = x.contiguous()
+    if type(x) is not _Tensor:  # new_empty makes tensors of the input's type
+        x = x.as_subclass(_Tensor)
     m = x.shape[0]
     blk = FORMATS[fmt]["block"]
     if k % blk:

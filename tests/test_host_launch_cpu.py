@@ -35,7 +35,9 @@ def test_calls_go_to_the_library_that_is_loaded_now(monkeypatch):
     for i in (1, 2):
         monkeypatch.setattr(_abi, "_lib", types.SimpleNamespace(komp_quant_q8_0=lambda *a, i=i: got.append(i) or 0))
         _abi.call("komp_quant_q8_0")
-        assert _abi.entry("komp_quant_q8_0")() == 0
+        monkeypatch.setattr(host, "_current_device", lambda: -1)
+        monkeypatch.setattr(host, "_raw_stream", lambda dev: None)
+        host._launch("komp_quant_q8_0", torch.zeros(1))
     assert got == [1, 1, 2, 2]
 
 
@@ -78,10 +80,11 @@ def test_launches_pass_the_tensors_devices_current_stream(monkeypatch):
         yield
         current[0] = before
 
-    def entry(name):
-        return lambda *a: log.append((name, current[0], a[-1])) or 0
+    class Library:
+        def __getattr__(self, name):
+            return lambda *a: log.append((name, current[0], a[-1])) or 0
 
-    monkeypatch.setattr(_abi, "entry", entry)
+    monkeypatch.setattr(_abi, "_lib", Library())
     monkeypatch.setattr(host, "_raw_stream", lambda dev: 1000 + dev)
     monkeypatch.setattr(host, "_current_device", lambda: current[0])
     monkeypatch.setattr(torch.cuda, "device", switched)
@@ -89,7 +92,7 @@ def test_launches_pass_the_tensors_devices_current_stream(monkeypatch):
     like = lambda t: t.as_subclass(OnDeviceOne)  # noqa: E731
     w, ws = like(torch.zeros((8, 512), dtype=torch.uint8)), like(torch.zeros((8, 32), dtype=torch.int16))
     x, xq, xd = like(torch.zeros((2, 1024))), like(torch.zeros((2, 1024), dtype=torch.int8)), like(torch.zeros((2, 32)))
-    monkeypatch.setattr(host, "_plain", lambda t: t)  # the device stays the fake one
+    monkeypatch.setattr(host, "_Tensor", OnDeviceOne)  # as plain tensors, so that the device stays the fake one
     for call, name in (
         (lambda: host.quantize("q4_0", x), "komp_quant_q8_0"),
         (lambda: host.gemv("q4_0", w, ws, xq, xd, 8, 1024), "komp_q4_0_gemv"),
